@@ -1199,6 +1199,114 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(DecodeArgs a) {
   merge_segment<D, kMaxG>(a, b, hk, seg, wave_of_tile(start, W, NW), wave_of_tile(last, W, NW), W, NW, lane);
 }
 
+// The same merge for few segments, whose pieces are many: one workgroup per
+// (segment, query head), its waves taking quarters of the pieces, their states
+// meeting in LDS. The merge above walks a segment's pieces on one wave, a
+// batch of rows per memory round trip; here every wave has its maxima, sums
+// and first kRows rows in one round trip. Bound by latency: prefix, then the
+// pieces, then the exchange. Kernel time, this merge against the one above
+// (H_kv 8, G 4, 60 k tokens in all), by segments:
+//   segments    8     16     32     64    128    192    256    384    512   1024
+//   D 128  us  4.5    4.8    4.0    4.2    4.7    4.7    4.4    5.2    6.0    9.2
+//   above     34.3   27.7   17.2    9.9    6.2    5.4    5.2    4.4    4.4    4.4
+//   D 64   us  6.4    6.2    4.4    4.0    4.0    4.1    4.5    5.4    6.0    9.6
+//   above     57.6   47.0   28.2   14.2    7.8    6.8    6.1    5.2    4.9    4.3
+template <int D>
+__global__ __launch_bounds__(64 * kWavesPerBlock) void decode_merge_wide_kernel(DecodeArgs a) {
+  constexpr int DPL = D >= 64 ? D / 64 : 1;
+  constexpr int kRows = 16;  // piece rows in flight per wave
+  __shared__ float so[kWavesPerBlock][D];
+  __shared__ float sm[kWavesPerBlock], sl[kWavesPerBlock];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.x;
+  const int seg = blockIdx.y;
+  const int G = a.group;
+  const int b = seg / a.hkv;
+  const int hk = seg - b * a.hkv;
+  const bool lane_in = D >= 64 || lane < D;
+  uint16_t *out = static_cast<uint16_t *>(a.out) + (int64_t)b * a.o_sb + (int64_t)(hk * G + h) * a.o_sh;
+  const int pb = a.ws_prefix[b];
+  const int nb = a.ws_prefix[b + 1] - pb;
+  const int64_t W = (int64_t)a.ws_prefix[a.batch] * a.hkv;
+  if (nb <= 0) {
+    if (threadIdx.x < a.head_dim) out[threadIdx.x] = 0;
+    return;
+  }
+  const int64_t NW = a.stream_waves;
+  const int64_t start = (int64_t)pb * a.hkv + (int64_t)hk * nb + a.seg_cost;  // as decode_merge_kernel
+  const int64_t last = (int64_t)pb * a.hkv + (int64_t)(hk + 1) * nb - 1;
+  // Pieces: with W >= NW every wave from the first tile's to the last tile's
+  // holds one; otherwise a wave holds at most one tile, and every tile is a piece.
+  const bool per_tile = W < NW;
+  const int w0 = (int)wave_of_tile(start, W, NW);
+  const int n = per_tile ? (int)(last - start) + 1 : (int)wave_of_tile(last, W, NW) - w0 + 1;
+  const int per = (n + kWavesPerBlock - 1) / kWavesPerBlock;
+  const int i0 = wave * per;
+  const int i1 = min(n, i0 + per);
+  float M = kNegInf, Ls = 0.f, acc[DPL];
+#pragma unroll
+  for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
+  for (int ib = i0; ib < i1; ib += 64) {
+    const int nk = min(64, i1 - ib);
+    const int i = ib + min(lane, nk - 1);  // lanes past the pieces repeat the last one, unused
+    const int slot = seg + (per_tile ? (int)((((uint32_t)(start + i) + 1) * (uint32_t)NW - 1) / (uint32_t)W) : w0 + i);
+    float ov[kRows][DPL];
+    auto load_rows = [&](int k0) {
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        const int64_t sk = __builtin_amdgcn_readlane(slot, min(k0 + u, nk - 1));
+#pragma unroll
+        for (int j = 0; j < DPL; ++j) ov[u][j] = lane_in ? a.ws_o[(sk * G + h) * D + lane + 64 * j] : 0.f;
+      }
+    };
+    const float m = a.ws_ml[((int64_t)slot * G + h) * 2];
+    const float l = a.ws_ml[((int64_t)slot * G + h) * 2 + 1];
+    load_rows(0);
+    const bool valid = lane < nk;
+    const float m_new = fmaxf(M, wave_max(m));  // finite: every piece holds a valid key
+    const float sc = __builtin_amdgcn_exp2f(M - m_new);
+    const float e = valid ? __builtin_amdgcn_exp2f(m - m_new) : 0.f;
+    Ls = Ls * sc + wave_sum(valid ? e * l : 0.f);
+#pragma unroll
+    for (int j = 0; j < DPL; ++j) acc[j] *= sc;
+    M = m_new;
+    for (int k0 = 0; k0 < nk; k0 += kRows) {
+      if (k0 > 0) load_rows(k0);
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        if (k0 + u < nk) {  // uniform
+          const float ek = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), k0 + u));
+#pragma unroll
+          for (int j = 0; j < DPL; ++j) acc[j] += ek * ov[u][j];
+        }
+      }
+    }
+  }
+  if (lane_in) {
+#pragma unroll
+    for (int j = 0; j < DPL; ++j) so[wave][lane + 64 * j] = acc[j];
+  }
+  if (lane == 0) {
+    sm[wave] = M;
+    sl[wave] = Ls;
+  }
+  __syncthreads();
+  if (threadIdx.x < a.head_dim) {  // head_dim <= D <= 128 < the block
+    float top = sm[0];
+#pragma unroll
+    for (int w = 1; w < kWavesPerBlock; ++w) top = fmaxf(top, sm[w]);  // wave 0 always holds a piece
+    float o = 0.f, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) {
+      const float f = __builtin_amdgcn_exp2f(sm[w] - top);
+      o += f * so[w][threadIdx.x];
+      sum += f * sl[w];
+    }
+    out[threadIdx.x] = f32_to_bf16_bits(sum > 0.f ? o / sum : 0.f);
+  }
+}
+
 // VALU path: fp32 caches (small models run in fp32, e.g. the reference
 // without autocast) and head dims the MFMA tiles do not take (not a multiple
 // of 16 bytes: of 8 bf16 or 16 fp8 values), any even head_dim <= 128. Fixed
@@ -1393,6 +1501,11 @@ hipError_t launch_mfma(const DecodeArgs &a, dim3 block, size_t lds_merge, hipStr
   return hipGetLastError();
 }
 
+// Segments up to which the wide merge runs: its segments x G workgroups of
+// four waves win while a segment has more pieces than the one-wave merge loads
+// in a round trip or two (both sides measured at decode_merge_wide_kernel).
+constexpr int64_t kMergeWideSegs = 256;
+
 template <int D, bool kFP8, bool kPad>
 hipError_t launch_stream(const DecodeArgs &a0, const DecodeAppend *ap, hipStream_t stream) {
   DecodeArgs a = a0;
@@ -1418,7 +1531,13 @@ hipError_t launch_stream(const DecodeArgs &a0, const DecodeAppend *ap, hipStream
   }
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  const dim3 mgrid((unsigned)((int64_t)a.batch * a.hkv));
+  const int64_t segs = (int64_t)a.batch * a.hkv;
+  if (segs <= kMergeWideSegs) {
+    hipLaunchKernelGGL((decode_merge_wide_kernel<D>), dim3(a.group, (unsigned)segs), dim3(64 * kWavesPerBlock), 0,
+                       stream, a);
+    return hipGetLastError();
+  }
+  const dim3 mgrid((unsigned)segs);
   if (a.group <= 4)
     hipLaunchKernelGGL((decode_merge_kernel<D, 4>), mgrid, dim3(64), 0, stream, a);
   else if (a.group <= 8)
