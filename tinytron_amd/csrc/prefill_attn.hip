@@ -7,18 +7,41 @@
 // append, get_kv, then SDPA with is_causal=True at past_len 0 or the mask
 // key_pos <= past_len + query_pos otherwise) for a ragged batch.
 //
-// One wave per (sequence b, KV head hk, NB consecutive blocks of qt = 16 / G
-// query tokens): the 16 columns of a block's MFMA B operand are the (token,
-// head) pairs n = tq * G + head, so each streamed K/V tile serves G heads x
-// NB * qt tokens (the tile's K fragments and its transposed V are reused by
-// all NB blocks). The key loop is the decode kernel's tile pipeline (K
-// fragments in registers, V through LDS, QK^T and PV on the matrix cores,
-// online softmax per column); column n masks the keys after its own position
-// (position 0 is valid for every column, so no row is ever empty).
+// One workgroup per (sequence b, KV head hk, 256 columns), a column being one
+// (query token, head of the group) pair: a wave owns 32 of them
+// (qt = 32 / G consecutive tokens) and walks the keys in tiles of 64 that
+// the whole workgroup shares through LDS. Every thread loads its 16-byte
+// pieces of the next tile's K and V into registers while the current tile is
+// computed and writes them to the other LDS buffer afterwards (one barrier a
+// tile); fp8 codes become bf16 on the way (exact), once per workgroup, so the
+// compute loop is one for both cache types.
 //
-// Workgroups are laid out so that all query blocks of one (sequence, KV
-// head) go to the same XCD (workgroup i runs on XCD i mod 8): the pair's
-// K/V, re-read by each of its blocks, stays in that XCD's L2.
+// Compute, per 32 keys and 32 columns, on v_mfma_f32_32x32x16_bf16:
+//   S^T = K q^T   A = K rows from LDS (16-byte reads), B = q (registers)
+//   softmax       a lane holds 16 keys of one column; the other 16 are in the
+//                 lane 32 away, so only a moving maximum crosses lanes
+//   O^T += V^T P^T  A = V read back transposed (ds_read_b64_tr_b16), B = P as
+//                 bf16 P_hi + P_lo (~16 mantissa bits: a single bf16 P misses
+//                 the 2e-3 absolute bound on short, cancelling rows). The order
+//                 of the 16 contracted keys is the one S^T's layout leaves in
+//                 each lane's registers, used for V as well: P needs no shuffle.
+//
+// Bound: the shared issue of VALU and matrix instructions. Per 32 x 32 block at
+// D 64 a wave issues ~125 VALU instructions (16 exponentials; the P split is 48,
+// the sums and the maxima 24) and 12 MFMAs; measured, 8 MFMAs and 64 FMAs of one
+// SIMD take 200 ns where either alone takes 145-160, so the two overlap by
+// half. With the same shape and timing-only loads of two fixed tiles the time
+// does not move: K/V traffic does not bind. Against one wave per 64 columns
+// streaming K/V for itself (K in registers, 16x16x32 MFMAs), kernel time:
+//   C5 prompts (64 x U[64, 2048], 32 / 8 heads)  D 64   bf16  843 -> 717 us
+//                                                       fp8  1019 -> 830 us
+//   4 x U[1024, 2048] after U[2048, 8192] cached D 128  fp8  1477 -> 1175 us
+//   8 x U[64, 4096]                              D 128  bf16  741 -> 601 us
+//   1 x 20 after 8000 cached                     D 128  bf16  409 -> 228 us
+//   6 x U[64, 2048], 32 / 4 heads                D 32   bf16  103 -> 70 us
+//
+// With many pairs, all query blocks of one (sequence, KV head) run on one XCD,
+// whose L2 keeps the pair's K/V for them (prefill_group).
 #include <algorithm>
 
 #include "attn_tiles.h"
@@ -28,355 +51,358 @@
 namespace tt {
 namespace {
 
-constexpr int kXcds = 8;
-// Tiles per page-table fetch and pipelined run: 8 here (16 measured 25 %
-// slower: NB column blocks per wave already make the unrolled body long).
-constexpr int kPrefillChunkTiles = 8;
 
-// QK^T and the online-softmax step of one 32-token tile for one column block
-// (16 (token, head) columns). Unlike the decode step this loop is bound by
-// VALU issue, so: bf16 scores become y = s * scale - m in one FMA; the causal
-// mask runs only on `edge` tiles (those reaching past the smallest limit of
-// the wave's columns: every other tile is whole for every column); the
-// maximum is the IEEE-754-2019 one (v_maximum3_f32, which needs no NaN
-// quieting of its inputs; no score is NaN). P enters PV as P_hi + P_lo
-// (two bf16 operands, ~16 mantissa bits: a single bf16 P misses the 2e-3
-// absolute bound on short, cancelling rows). The running max is lazy: a
-// column's reference max st.m moves only when the tile's max exceeds it by
-// more than kLazyMax (log2 units), so P <= 2^kLazyMax (fp32 O and l and the
-// bf16 P halves have the range) and most tiles need no rescale at all.
-// Returns whether any column of the wave moved its max; then the caller
-// rescales O by `alpha` (this column's exp2(m_old - m_new), 1 for columns
-// that kept theirs, 0 on the first tile, whose key 0 is valid for every
-// column).
-constexpr float kLazyMax = 8.0f;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x4t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Waves per workgroup (32 columns each) and the waves per SIMD that the
+// registers must leave room for. bf16 at tile width <= 64 fits 128 registers: two
+// workgroups of 8 waves per CU. Width 128 (q and O alone take 96 registers)
+// runs one; fp8 at width 64 (the scales' registers) three of 4 waves. Wider
+// workgroups read the pair's K/V from L2 less often; more waves per SIMD run
+// one's softmax beside another's MFMAs. Measured (C5 prompts, D 64): 8 waves x
+// two workgroups 717 us, two 32-column blocks a wave at two waves per SIMD 750,
+// 4 waves x three 786; (prefix 2k-8k, fp8, D 128): 8 waves 1154-1190 us, 4
+// waves x two 1171-1292, tiles of 128 keys 1289.
 template <int D, bool kFP8>
-__device__ __forceinline__ bool qk_softmax_pf(float scale_log2, const f32x4 (&kc)[2], bool edge, int t0, int lim,
-                                              int lane, const Tile<D, kFP8> &tile, const bf16x8 (&qf)[D / 32],
-                                              WaveState<D, kFP8> &st, float &alpha, bf16x8 &pa_hi, bf16x8 &pa_lo) {
-  using TR = KVTraits<kFP8>;
-  constexpr int NDB = D / 32;
-  const int g = lane >> 4;
-  // S^T[token][column]: lane (n + 16g), reg r = token t0 + 16*tt + 4g + r, column n.
-  f32x4 S[2];
+struct PrefillShape {
+  static constexpr int NW = D == 64 && kFP8 ? 4 : 8;
+  static constexpr int kOcc = D == 128 ? 2 : D == 64 && kFP8 ? 3 : 4;
+  static constexpr int kKeys = 64;  // keys per LDS tile
+  static constexpr int kThreads = 64 * NW;
+  static constexpr int kRowBytes = 2 * D;           // LDS rows hold bf16
+  static constexpr int kTileBytes = kKeys * kRowBytes;
+  // LDS: K[2] | V[2] | fp8: K scales [2][64], V scales [2][64]
+  static constexpr int kScaleAt = 4 * kTileBytes;
+  static constexpr int kLds = kScaleAt + (kFP8 ? 4 * kKeys * 4 : 0);
+};
+
+// 16-byte chunk c of row r lies at chunk c ^ swizzle(r) of the row, so that
+// 16 rows at one chunk (a K read's 16 lanes) resp. 4 rows of 64 bytes (a
+// transposing V read's 32 lanes) fall on distinct banks.
+template <int D>
+__device__ __forceinline__ int k_swizzle(int r) {
+  return D == 128 ? r & 15 : D == 64 ? (r >> 1) & 7 : (r >> 2) & 3;
+}
+template <int D>
+__device__ __forceinline__ int v_swizzle(int r) {
+  return D == 128 ? 4 * (r & 3) : D == 64 ? 4 * ((r >> 1) & 1) : 0;
+}
+
+// This thread's share of one tile on its way from the cache to LDS: N of the
+// tile's 16-byte chunks, K's rows first, then V's.
+template <int D, bool kFP8>
+struct Staged {
+  using SH = PrefillShape<D, kFP8>;
+  static constexpr int kChunks = D * (kFP8 ? 1 : 2) / 16;  // of a cached row
+  static constexpr int kHalf = SH::kKeys * kChunks;        // K's chunks
+  static constexpr int N = 2 * kHalf / SH::kThreads;
+  static_assert(N * SH::kThreads == 2 * kHalf && kHalf % 64 == 0 && 64 / kChunks <= 16, "a wave: K or V, one block");
+  u32x4 x[N];
+  float scale[N];  // fp8: the row's scale, in the thread that holds the row's first chunk
+  static __device__ __forceinline__ bool is_v(int j) {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x + j * SH::kThreads) >= kHalf;
+  }
+  static __device__ __forceinline__ int row(int j) {
+    return (threadIdx.x + j * SH::kThreads) % kHalf / kChunks;
+  }
+  static __device__ __forceinline__ int chunk() { return threadIdx.x % kChunks; }
+};
+
+// Issue the loads of the tile at key t0. `entry` holds, one per lane, the
+// page-table entries of pages pbase.. (see stream_block_addr); rows past L and
+// chunks past a padded row's end read zero (the buffer range).
+template <int D, bool kFP8, bool kPad>
+__device__ __forceinline__ void stage_load(const DecodeArgs &a, int b, int hk, int L, int entry, int pbase, int t0,
+                                           Staged<D, kFP8> &st) {
+  using ST = Staged<D, kFP8>;
+  constexpr int E = KVTraits<kFP8>::kElemBytes;
+  const int hd = row_len<D, kPad>(a);
+  const int c = ST::chunk();
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt) {
-    S[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < NDB; ++s) {
-      const int u = s / TR::kStepsPerFrag;
-      S[tt] = mfma_bf16(TR::step(tile.k[tt][u], s % TR::kStepsPerFrag), qf[s], S[tt]);
+  for (int j = 0; j < ST::N; ++j) {
+    const int row = ST::row(j);
+    const int blk = __builtin_amdgcn_readfirstlane(t0 / 16 + row / 16);
+    int64_t elem;
+    int rows;
+    stream_block_addr<D, kPad>(a, b, hk, L, entry, pbase, blk, elem, rows);
+    const char *base = static_cast<const char *>(ST::is_v(j) ? a.v_cache : a.k_cache) + elem * E;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(base), (short)0, rows * hd * E, kBufferFlags);
+    const int off = (kPad && 16 * c >= hd * E) ? 0x7ffffff0 : (row & 15) * hd * E + 16 * c;
+    st.x[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+    if constexpr (kFP8) {
+      // the block starts a 16-row scale group (the host checks the strides)
+      const float *sc = (ST::is_v(j) ? a.v_scale : a.k_scale) + fp8_scale_index(scale_row<D, kPad>(a, elem));
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(sc), (short)0, rows * 4, kBufferFlags);
+      st.scale[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, c == 0 ? 4 * (row & 15) : 0x7ffffff0, 0, 0));
     }
   }
-  // x: raw scores (bf16) or scores in log2 units (fp8: K scale x softmax scale)
-  float x[8];
+}
+
+// The staged pieces into LDS buffer `buf` as bf16 rows.
+template <int D, bool kFP8>
+__device__ __forceinline__ void stage_store(const DecodeArgs &a, const Staged<D, kFP8> &st, char *lds, int buf) {
+  using ST = Staged<D, kFP8>;
+  using SH = PrefillShape<D, kFP8>;
+  const int c = ST::chunk();
 #pragma unroll
-  for (int i = 0; i < 8; ++i) x[i] = kFP8 ? S[i >> 2][i & 3] * kc[i >> 2][i & 3] : S[i >> 2][i & 3];
-  if (edge) {
+  for (int j = 0; j < ST::N; ++j) {
+    const int row = ST::row(j);
+    const bool v = ST::is_v(j);  // uniform
+    char *dst = lds + (buf + (v ? 2 : 0)) * SH::kTileBytes + row * SH::kRowBytes;
+    const int f = v ? v_swizzle<D>(row) : k_swizzle<D>(row);
+    if constexpr (kFP8) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = t0 + 16 * (i >> 2) + 4 * g + (i & 3) < lim ? x[i] : kNegInf;
-  }
-  const auto mx2 = [](float u, float v) { return __builtin_elementwise_maximum(u, v); };
-  // nested pairs fold into three-input v_maximum3_f32 (four instructions for eight values)
-  float mx = mx2(mx2(mx2(mx2(x[0], x[1]), x[2]), mx2(mx2(x[3], x[4]), x[5])), mx2(x[6], x[7]));
-  // The reference max moves only past the slack (always on the first tile:
-  // st.m = -inf). A column moves iff one of its four lanes' own maxima is past
-  // it (scaling by scale > 0 and rounding keep the order, -inf stays -inf), so
-  // the maxima across the lane groups need only be formed when some column
-  // moves (same results).
-  const bool lane_past = (kFP8 ? mx : mx * scale_log2) > st.m + kLazyMax;
-  const bool rescale = __builtin_amdgcn_ballot_w64(lane_past) != 0;  // wave-uniform
-  alpha = 1.0f;
-  float m_new = st.m;
-  if (rescale) {  // across the four lane groups (lanes n, n+16, n+32, n+48 hold column n)
-    const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-    mx = mx2(__uint_as_float(p16[0]), __uint_as_float(p16[1]));
-    const auto p32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-    mx = mx2(__uint_as_float(p32[0]), __uint_as_float(p32[1]));
-    if constexpr (!kFP8) mx *= scale_log2;
-    m_new = mx > st.m + kLazyMax ? mx : st.m;
-    alpha = __builtin_amdgcn_exp2f(st.m - m_new);
-    st.m = m_new;
-  }
-  float p[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    p[i] = __builtin_amdgcn_exp2f(kFP8 ? x[i] - m_new : __builtin_fmaf(x[i], scale_log2, -m_new));
-  if constexpr (kFP8) {  // bf16: the column sums come from the matrix cores (see pv_block)
-    const float psum = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-    st.l = rescale ? __builtin_fmaf(st.l, alpha, psum) : st.l + psum;
-  }
-  if constexpr (kFP8) {
-    // fold the per-token V scale into P; on edge tiles masked tokens stay
-    // exactly 0 (select: a scale slot past the end may hold anything)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float pv = p[i] * tile.vs[i >> 2][i & 3];
-      p[i] = edge ? (p[i] == 0.f ? 0.f : pv) : pv;
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<bf16x8 *>(dst + 16 * ((2 * c + h) ^ f)) =
+            fp8x8_to_bf16x8(u32x2{st.x[j][2 * h], st.x[j][2 * h + 1]});
+      if (c == 0)  // K scales carry the softmax scale: scores come out in log2 units
+        reinterpret_cast<float *>(lds + SH::kScaleAt)[(buf + (v ? 2 : 0)) * SH::kKeys + row] =
+            v ? st.scale[j] : st.scale[j] * a.scale_log2;
+    } else {
+      *reinterpret_cast<u32x4 *>(dst + 16 * (c ^ f)) = st.x[j];
     }
   }
+}
+
+// Lazy running maximum: a column's reference moves only when a tile's maximum
+// exceeds it by more than kLazyMax (log2 units), so P <= 2^kLazyMax (fp32 O and
+// l and the bf16 P halves have the range) and most tiles need no rescale.
+constexpr float kLazyMax = 8.0f;
+
+// p (one lane's 8 softmax values of a contraction step) as bf16 P_hi + P_lo:
+// P_lo = bf16(p - P_hi), the difference exact in fp32.
+__device__ __forceinline__ void split_p(const float (&p)[8], bf16x8 &hi, bf16x8 &lo) {
   const f32x8 pv = {p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]};
-  pa_hi = __builtin_convertvector(pv, bf16x8);
-  // P_hi back in fp32 straight from the packed halves (element 2i is the low half of word i)
-  const u32x4 hw = __builtin_bit_cast(u32x4, pa_hi);
-  f32x8 hf;
+  hi = __builtin_convertvector(pv, bf16x8);
+  f32x8 rem;
+  const u32x4 hw = __builtin_bit_cast(u32x4, hi);  // P_hi back in fp32 from the packed halves
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    hf[2 * i] = __uint_as_float(hw[i] << 16);
-    hf[2 * i + 1] = __uint_as_float(hw[i] & 0xffff0000u);
+    rem[2 * i] = p[2 * i] - __uint_as_float(hw[i] << 16);
+    rem[2 * i + 1] = p[2 * i + 1] - __uint_as_float(hw[i] & 0xffff0000u);
   }
-  pa_lo = __builtin_convertvector(pv - hf, bf16x8);  // P - P_hi exact in fp32
-  return rescale;
+  lo = __builtin_convertvector(rem, bf16x8);
 }
 
-// PV of one tile for one column block, accumulated transposed: Oᵀ = Vᵀ Pᵀ,
-// with the V block as the A operand and P_hi + P_lo as B (the same
-// registers as in P V: lane (n + 16g) holds V[tokens of group g][d n] and
-// P[column n][tokens of group g]). Lane (n + 16g) then holds Oᵀ[d][column n]
-// for d = o_col_d(c, 4g + r): every O value of a lane belongs to its own
-// column, so the rescale by alpha needs no cross-lane traffic, and each
-// block's four values are consecutive head_dim entries. bf16 caches also
-// accumulate the softmax denominators here: an all-ones A block gives every
-// column's sum of P_hi + P_lo in each of its lanes (two MFMAs instead of
-// eight VALU adds per block and tile, in a loop bound by VALU issue; fp8 P
-// carries the V scales, so fp8 sums on the VALU). `vb` are the tile's V
-// blocks (v_block), converted once for all column blocks.
-template <int D, bool kFP8>
-__device__ __forceinline__ void pv_block(const bf16x8 (&vb)[D / 16], bf16x8 pa_hi, bf16x8 pa_lo,
-                                         WaveState<D, kFP8> &st, f32x4 &lsum) {
-#pragma unroll
-  for (int c = 0; c < D / 16; ++c) {
-    st.o[c] = mfma_bf16(vb[c], pa_hi, st.o[c]);
-    st.o[c] = mfma_bf16(vb[c], pa_lo, st.o[c]);
-  }
-  if constexpr (!kFP8) {
-    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-    lsum = mfma_bf16(ones, pa_hi, lsum);
-    lsum = mfma_bf16(ones, pa_lo, lsum);
-  }
-}
-
-// Column blocks per wave and workgroups per CU. bf16 at head_dim 128 runs
-// 4 blocks at one workgroup per CU (up to 512 registers a wave): the K
-// fragments and transposed V of a tile then feed twice the MFMA work per
-// byte read, which pays more than the second workgroup's latency hiding.
-// fp8 keeps 2 blocks at two workgroups per CU at 128: its dequantisation is
-// VALU work that needs the second workgroup to hide.
-template <int D, bool kFP8>
-constexpr int prefill_blocks() {
-  return D <= 64 ? 4 : (kFP8 ? 2 : 4);
-}
-
-template <int D, bool kFP8>
-constexpr int prefill_wgs_per_cu() {
-  return (D == 128 && !kFP8) ? 1 : 2;
-}
-
-template <int D, bool kFP8, int NB, bool kPad>
-__global__ __launch_bounds__(256, (prefill_wgs_per_cu<D, kFP8>())) void prefill_attn_kernel(PrefillArgs a) {
-  using TR = KVTraits<kFP8>;
+template <int D, bool kFP8, bool kPad>
+__global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D, kFP8>::kOcc)) void prefill_attn_kernel(PrefillArgs a) {
+  using SH = PrefillShape<D, kFP8>;
+  constexpr int kKeys = SH::kKeys;
+  constexpr int NU = kKeys / 32;
+  const auto mx2 = [](float u, float v) { return __builtin_elementwise_maximum(u, v); };
   const int hd = row_len<D, kPad>(a);
-  constexpr int NDB = D / 32;
-  constexpr int NU = Tile<D, kFP8>::NU;
-  constexpr int kKLoads = 2 * NU + (kFP8 ? 4 : 0);
-  constexpr int kVAll = kWavesPerBlock * Tile<D, kFP8>::kVBytes;
-  extern __shared__ char smem_v[];
+  __shared__ __attribute__((aligned(16))) char lds[SH::kLds];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int i = threadIdx.x; i < kVAll / 16; i += 64 * kWavesPerBlock)  // the block size (not a dispatch load)
-    reinterpret_cast<u32x4 *>(smem_v)[i] = u32x4{0u, 0u, 0u, 0u};
-  __syncthreads();
+  const int half = lane >> 5;
+  const int n = lane & 31;
 
-  // workgroup -> (XCD, slot on that XCD) -> (pair, its k-th workgroup); the
-  // longest (last) query blocks of a pair go first. a.nq counts groups of NB
-  // blocks here.
-  const int xcd = blockIdx.x % kXcds;
-  const int slot = blockIdx.x / kXcds;
-  const int pair = (slot / a.wg_per_pair) * kXcds + xcd;
-  if (pair >= a.batch * a.hkv) return;
-  const int qgrp = a.nq - 1 - ((slot % a.wg_per_pair) * kWavesPerBlock + wave);
-  if (qgrp < 0) return;
+  int pair, grp;
+  if (!prefill_group(a, pair, grp)) return;
   const int b = pair / a.hkv;
   const int hk = pair - b * a.hkv;
   const int nb = a.new_lens != nullptr ? min(max(a.new_lens[b], 0), a.num_new) : a.num_new;
-  const int t_first = qgrp * a.qt * NB;
-  if (t_first >= nb) return;
+  const int wg_tokens = a.qt * SH::NW;
+  if (grp * wg_tokens >= nb) return;
   const int pos0 = a.positions[b];
-  const int t_end = min(t_first + a.qt * NB, nb);
-  // keys the group needs: 0 .. pos0 + t_end - 1, never past the host's bound (the page table's reach)
-  const int L = __builtin_amdgcn_readfirstlane(min(pos0 + t_end, a.max_len));
+  // keys of the workgroup resp. the wave: 0 .. its last token, never past the host's bound (the page table's reach)
+  const int L = __builtin_amdgcn_readfirstlane(min(pos0 + min((grp + 1) * wg_tokens, nb), a.max_len));
   if (pos0 < 0 || L <= 0) return;
-  // smallest key limit of the wave's valid columns (its first token's): tiles
-  // below it are whole for every column and skip the mask
+  const int t_first = grp * wg_tokens + wave * a.qt;
+  const int t_end = min(t_first + a.qt, nb);
+  const int Lw = t_first < nb ? __builtin_amdgcn_readfirstlane(min(pos0 + t_end, L)) : 0;
+  // smallest key limit of the wave's valid columns (its first token's): key
+  // ranges below it are whole for every column and skip the mask
   const int lim_min = __builtin_amdgcn_readfirstlane(min(pos0 + t_first + 1, L));
 
   const int G = a.group;
-  const int n = lane & 15;
-  const int g = lane >> 4;
   const int tq = n / G;
   const int head = n - tq * G;
-  int lim[NB];
-  bf16x8 qf[NB][NDB];
-  const uint16_t *q = static_cast<const uint16_t *>(a.q);
+  const int tok = t_first + tq;
+  const bool col_valid = tq < a.qt && tok < t_end;
+  const int lim = col_valid ? min(pos0 + tok + 1, L) : 1;  // keys this column may see
+  bf16x8 qf[D / 16];
+  const uint16_t *q = static_cast<const uint16_t *>(a.q) + (int64_t)b * a.q_sb + (int64_t)(hk * G + head) * a.q_sh +
+                      (int64_t)tok * a.q_st;
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    const int tb = t_first + j * a.qt;
-    const bool col_valid = tq < a.qt && tb + tq < t_end;
-    lim[j] = col_valid ? min(pos0 + tb + tq + 1, L) : 1;  // keys this column may see
-    const int64_t qrow = (int64_t)b * a.q_sb + (int64_t)(hk * G + head) * a.q_sh + (int64_t)(tb + tq) * a.q_st;
-#pragma unroll
-    for (int s = 0; s < NDB; ++s) {
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (col_valid && (!kPad || TR::q_offset(s, g) < hd)) v = *reinterpret_cast<const u32x4 *>(q + qrow + TR::q_offset(s, g));
-      qf[j][s] = __builtin_bit_cast(bf16x8, v);
-    }
+  for (int s = 0; s < D / 16; ++s) {
+    const int d = 16 * s + 8 * half;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (col_valid && (!kPad || d < hd)) v = *reinterpret_cast<const u32x4 *>(q + d);
+    qf[s] = __builtin_bit_cast(bf16x8, v);
   }
-  bf16x8 ident16[2];
-  u32x2 ident8[2];
-  make_identity(lane, ident16, ident8);
-  WaveState<D, kFP8> st[NB];
+  f32x16 o[D / 32];
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int c = 0; c < D / 32; ++c)
 #pragma unroll
-    for (int c = 0; c < 2 * NDB; ++c) st[j].o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    st[j].m = kNegInf;
-    st[j].l = 0.f;
-  }
-  f32x4 lsum[NB];  // bf16: every element holds the lane's column sum of P (rescaled with O)
-#pragma unroll
-  for (int j = 0; j < NB; ++j) lsum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < 16; ++r) o[c][r] = 0.f;
+  float m = kNegInf, l = 0.f;  // the column's reference maximum (log2 units); this lane's part of its sum
 
-  char *vlds = smem_v + wave * Tile<D, kFP8>::kVBytes;
-  const int ntiles = (L + kTileTokens - 1) / kTileTokens;
-  // Same chunked pipeline as the decode kernel (K(k+1) | QK, softmax |
-  // wait V(k), read V(k) | V(k+1) | PV), with explicit vmcnt counts.
-  for (int c0 = 0; c0 < ntiles; c0 += kPrefillChunkTiles) {
-    const int c1 = min(ntiles, c0 + kPrefillChunkTiles);
-    int entry = 0, pbase = 0;
+  // page-table entries of 64 pages (>= 16 tiles) at a time, one per lane
+  const int tiles = (L + kKeys - 1) / kKeys;
+  const int last_page = (L - 1) >> a.page_shift;
+  int entry = 0, pbase = 0;
+  auto fetch_entries = [&](int tile) {
     if (a.page_table != nullptr) {
-      pbase = (kTileTokens * c0) >> a.page_shift;
-      const int last = (L - 1) >> a.page_shift;
-      entry = a.page_table[(int64_t)b * a.max_pages + min(pbase + lane, last)];
+      pbase = (kKeys * tile) >> a.page_shift;
+      entry = a.page_table[(int64_t)b * a.max_pages + min(pbase + lane, last_page)];
     }
-    Tile<D, kFP8> buf[2];
-    int64_t e0, e1;
-    int r0, r1;
-    stream_block_addr<D, kPad>(a, b, hk, L, entry, pbase, 2 * c0, e0, r0);
-    stream_block_addr<D, kPad>(a, b, hk, L, entry, pbase, 2 * c0 + 1, e1, r1);
-    load_k_block<D, kFP8, kPad>(a, e0, r0, lane, buf[0].k[0], buf[0].ks[0], buf[0].vs[0]);
-    load_k_block<D, kFP8, kPad>(a, e1, r1, lane, buf[0].k[1], buf[0].ks[1], buf[0].vs[1]);
+  };
+  Staged<D, kFP8> st;
+  fetch_entries(0);
+  stage_load<D, kFP8, kPad>(a, b, hk, L, entry, pbase, 0, st);
+  stage_store<D, kFP8>(a, st, lds, 0);
+  __syncthreads();
+
+  // this lane's K row and V rows (see k_swizzle / v_swizzle); XORed with the
+  // chunk of a k step resp. a 32-column block
+  const int ka0 = n * SH::kRowBytes + 16 * (half ^ k_swizzle<D>(n));
+  const int vj = (lane >> 2) & 3, vq = lane & 3;  // key 4 half + vj, columns 4 vq .. + 3 of a 16-column group
+  const int va0 = (4 * half + vj) * SH::kRowBytes +
+                  16 * (v_swizzle<D>(4 * half + vj) + 2 * ((lane >> 4) & 1) + (vq >> 1)) + 8 * (vq & 1);
+  for (int i = 0; i < tiles; ++i) {
+    const bool more = i + 1 < tiles;
+    if (more) {
+      if ((kKeys * (i + 1)) % 1024 == 0) fetch_entries(i + 1);
+      stage_load<D, kFP8, kPad>(a, b, hk, L, entry, pbase, kKeys * (i + 1), st);
+    }
     __builtin_amdgcn_sched_barrier(0);
-    load_v_block_lds<D, kFP8, kPad>(a, e0, r0, lane, vlds);
-    load_v_block_lds<D, kFP8, kPad>(a, e1, r1, lane, vlds + NU * 1024);
-    __builtin_amdgcn_sched_barrier(0);
+    const char *kb = lds + (i & 1) * SH::kTileBytes;
+    const char *vb = kb + 2 * SH::kTileBytes;
+    const float *sc = reinterpret_cast<const float *>(lds + SH::kScaleAt) + (i & 1) * kKeys;
+    const int t0 = kKeys * i;
+    if (t0 < Lw) {  // uniform
+      f32x16 S[NU];
 #pragma unroll
-    for (int k = 0; k < kPrefillChunkTiles; ++k) {
-      const int it = c0 + k;
-      if (it >= c1) break;  // uniform
-      if (k + 1 < kPrefillChunkTiles) {
-        stream_block_addr<D, kPad>(a, b, hk, L, entry, pbase, 2 * it + 2, e0, r0);
-        stream_block_addr<D, kPad>(a, b, hk, L, entry, pbase, 2 * it + 3, e1, r1);
-        Tile<D, kFP8> &nx = buf[(k + 1) & 1];
-        load_k_block<D, kFP8, kPad>(a, e0, r0, lane, nx.k[0], nx.ks[0], nx.vs[0]);
-        load_k_block<D, kFP8, kPad>(a, e1, r1, lane, nx.k[1], nx.ks[1], nx.vs[1]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      const int t0 = kTileTokens * it;
-      const bool edge = t0 + kTileTokens > lim_min;  // uniform
-      f32x4 kc[2] = {};
-      if constexpr (kFP8) {
-        kc[0] = buf[k & 1].ks[0] * a.scale_log2;
-        kc[1] = buf[k & 1].ks[1] * a.scale_log2;
-      }
-      // Every column block's QKᵀ and softmax go before the wait for V(k) (time
-      // for its DMA to land; moving some blocks after it, to overlap their
-      // softmax with other blocks' PV, measured no faster with a bf16 cache and
-      // far slower with fp8 at head_dim 128). After the V read, each block's
-      // rescale and PV follow with no scheduling barrier between blocks.
-      bf16x8 pa_hi[NB], pa_lo[NB];
-      float alpha[NB];
-      bool rescale[NB];
+      for (int u = 0; u < NU; ++u)
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
-        rescale[j] = qk_softmax_pf<D, kFP8>(a.scale_log2, kc, edge, t0, lim[j], lane, buf[k & 1], qf[j], st[j],
-                                            alpha[j], pa_hi[j], pa_lo[j]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (k + 1 < kPrefillChunkTiles)
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(kKLoads));
-      else
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-      VRegs<D, kFP8> vr;
-      read_v<D, kFP8>(vlds, lane, vr);
-      __builtin_amdgcn_s_waitcnt(kLgkmcntZero);
-      __builtin_amdgcn_sched_barrier(0);
-      if (k + 1 < kPrefillChunkTiles && it + 1 < c1) {
-        load_v_block_lds<D, kFP8, kPad>(a, e0, r0, lane, vlds);
-        load_v_block_lds<D, kFP8, kPad>(a, e1, r1, lane, vlds + NU * 1024);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      bf16x8 vb[D / 16];
+        for (int r = 0; r < 16; ++r) S[u][r] = 0.f;
 #pragma unroll
-      for (int c = 0; c < D / 16; ++c) vb[c] = v_block<D, kFP8>(vr, c, ident8);
+      for (int s = 0; s < D / 16; ++s)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        // every Oᵀ value of a lane is in the lane's own column: its own alpha
-        if (rescale[j]) {  // uniform
-#pragma unroll
-          for (int c = 0; c < 2 * NDB; ++c) st[j].o[c] *= alpha[j];
-          if constexpr (!kFP8) lsum[j] *= alpha[j];
+        for (int u = 0; u < NU; ++u) {  // two independent chains
+          const bf16x8 kf = *reinterpret_cast<const bf16x8 *>(kb + 32 * u * SH::kRowBytes + (ka0 ^ (32 * s)));
+          S[u] = mfma32(kf, qf[s], S[u]);
         }
-        pv_block<D, kFP8>(vb, pa_hi[j], pa_lo[j], st[j], lsum[j]);
+      if constexpr (kFP8) {  // K scales (times the softmax scale: log2 units)
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const f32x4 kc = *reinterpret_cast<const f32x4 *>(sc + 32 * u + 8 * x + 4 * half);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[u][4 * x + r] *= kc[r];
+          }
       }
+      if (t0 + kKeys > lim_min) {  // uniform: a tile that some column sees only in part
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = t0 + 32 * u + 8 * (r >> 2) + (r & 3) + 4 * half;
+            S[u][r] = key < lim ? S[u][r] : kNegInf;
+          }
+      }
+      float mx = S[0][0];  // nested pairs fold into three-input maxima
+#pragma unroll
+      for (int r = 1; r < 16 * NU - 1; r += 2) mx = mx2(mx2(mx, S[r >> 4][r & 15]), S[(r + 1) >> 4][(r + 1) & 15]);
+      mx = mx2(mx, S[NU - 1][15]);
+      // A column moves iff one of its two lanes' own maxima is past its
+      // reference (always on the first tile: m = -inf, key 0 valid); only then
+      // are they combined and O rescaled.
+      if (__builtin_amdgcn_ballot_w64((kFP8 ? mx : mx * a.scale_log2) > m + kLazyMax) != 0) {  // uniform
+        const auto p32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = mx2(__uint_as_float(p32[0]), __uint_as_float(p32[1]));
+        if constexpr (!kFP8) mx *= a.scale_log2;
+        const float m_new = mx > m + kLazyMax ? mx : m;
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        l *= alpha;
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c) o[c] *= alpha;
+      }
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          bf16x8 vf[D / 32];
+#pragma unroll
+          for (int c = 0; c < D / 32; ++c) {
+            bf16x4t part[2];
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+              part[w] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4t *)(
+                  vb + (32 * u + 16 * t + 8 * w) * SH::kRowBytes + (va0 ^ (64 * c))));
+            vf[c] = bf16x8{part[0][0], part[0][1], part[0][2], part[0][3],
+                           part[1][0], part[1][1], part[1][2], part[1][3]};
+          }
+          float p[8];
+#pragma unroll
+          for (int r = 0; r < 8; ++r)
+            p[r] = __builtin_amdgcn_exp2f(kFP8 ? S[u][8 * t + r] - m
+                                               : __builtin_fmaf(S[u][8 * t + r], a.scale_log2, -m));
+          l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+          if constexpr (kFP8) {  // fold the V scales in; a row past the end has scale and P zero
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+              const f32x4 vc = *reinterpret_cast<const f32x4 *>(sc + 2 * kKeys + 32 * u + 16 * t + 8 * x + 4 * half);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) p[4 * x + r] *= vc[r];
+            }
+          }
+          bf16x8 hi, lo;
+          split_p(p, hi, lo);
+#pragma unroll
+          for (int c = 0; c < D / 32; ++c) o[c] = mfma32(vf[c], hi, o[c]);
+#pragma unroll
+          for (int c = 0; c < D / 32; ++c) o[c] = mfma32(vf[c], lo, o[c]);
+        }
     }
-    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_sched_barrier(0);
+    // the other buffer's readers are done since the last barrier
+    if (more) stage_store<D, kFP8>(a, st, lds, (i + 1) & 1);
+    __syncthreads();
   }
 
-  // normalise and write: lane (n + 16g) holds column n's head_dim entries
-  // o_col_d(c, 4g) .. + 3 of every block c
-  uint16_t *out = static_cast<uint16_t *>(a.out);
+  // normalise and write: the lane's column, head_dim entries 32 c + 8 i + 4 half .. + 3
+  const float sum = l + __shfl_xor(l, 32, 64);
+  const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+  if (!col_valid) return;
+  uint16_t *out = static_cast<uint16_t *>(a.out) + (int64_t)b * a.o_sb + (int64_t)tok * a.o_st +
+                  (int64_t)(hk * G + head) * a.o_sh;
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    const int tb = t_first + j * a.qt;
-    float l = lsum[j][0];
-    if constexpr (kFP8) {
-      l = st[j].l;
-      l += __shfl_xor(l, 16, 64);
-      l += __shfl_xor(l, 32, 64);
-    }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
-    if (tq < a.qt && tb + tq < t_end) {
-      const int64_t orow = (int64_t)b * a.o_sb + (int64_t)(tb + tq) * a.o_st + (int64_t)(hk * G + head) * a.o_sh;
+  for (int c = 0; c < D / 32; ++c)
 #pragma unroll
-      for (int c = 0; c < 2 * NDB; ++c) {
-        const int d0 = o_col_d<kFP8>(c, 4 * g);
-        if (kPad && d0 >= hd) continue;  // columns past head_dim (hd is a multiple of 8)
-        const uint2 w = make_uint2(pack_bf16x2(st[j].o[c][0] * inv, st[j].o[c][1] * inv),
-                                   pack_bf16x2(st[j].o[c][2] * inv, st[j].o[c][3] * inv));
-        if (a.vec_out) {
-          *reinterpret_cast<uint2 *>(out + orow + d0) = w;
-        } else {
-          out[orow + d0] = (uint16_t)w.x;
-          out[orow + d0 + 1] = (uint16_t)(w.x >> 16);
-          out[orow + d0 + 2] = (uint16_t)w.y;
-          out[orow + d0 + 3] = (uint16_t)(w.y >> 16);
-        }
+    for (int i = 0; i < 4; ++i) {
+      const int d0 = 32 * c + 8 * i + 4 * half;
+      if (kPad && d0 >= hd) continue;  // columns past head_dim (hd is a multiple of 8)
+      const uint2 w = make_uint2(pack_bf16x2(o[c][4 * i] * inv, o[c][4 * i + 1] * inv),
+                                 pack_bf16x2(o[c][4 * i + 2] * inv, o[c][4 * i + 3] * inv));
+      if (a.vec_out) {
+        *reinterpret_cast<uint2 *>(out + d0) = w;
+      } else {
+        out[d0] = (uint16_t)w.x;
+        out[d0 + 1] = (uint16_t)(w.x >> 16);
+        out[d0 + 2] = (uint16_t)w.y;
+        out[d0 + 3] = (uint16_t)(w.y >> 16);
       }
     }
-  }
 }
 
 template <int D, bool kFP8, bool kPad>
 hipError_t launch_d(const PrefillArgs &a0, hipStream_t stream) {
-  constexpr int NB = prefill_blocks<D, kFP8>();
+  using SH = PrefillShape<D, kFP8>;
   PrefillArgs a = a0;
-  a.nq = (a0.nq + NB - 1) / NB;  // groups of NB query blocks
-  a.wg_per_pair = (a.nq + kWavesPerBlock - 1) / kWavesPerBlock;
-  const int64_t pairs = (int64_t)a.batch * a.hkv;
-  const int64_t slots = (pairs + kXcds - 1) / kXcds * a.wg_per_pair;
-  const int64_t grid = slots * kXcds;
-  const size_t lds = (size_t)kWavesPerBlock * Tile<D, kFP8>::kVBytes;
-  hipLaunchKernelGGL((prefill_attn_kernel<D, kFP8, NB, kPad>), dim3((unsigned)grid), dim3(64 * kWavesPerBlock), lds,
-                     stream, a);
+  a.qt = 32 / a.group;  // group <= 16
+  const int wg_tokens = a.qt * SH::NW;
+  a.wg_per_pair = (a.num_new + wg_tokens - 1) / wg_tokens;
+  hipLaunchKernelGGL((prefill_attn_kernel<D, kFP8, kPad>), dim3((unsigned)prefill_grid(a)), dim3(SH::kThreads), 0, stream,
+                     a);
   return hipGetLastError();
 }
 
