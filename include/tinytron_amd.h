@@ -351,6 +351,17 @@ int tt_prefill_attn_bf16(const void *q, const int64_t q_strides[3],
                          int64_t batch, int64_t num_new, int64_t num_q_heads, int64_t num_kv_heads,
                          int64_t head_dim, int64_t page_size, float sm_scale, tt_stream_t stream);
 
+/* As tt_prefill_attn_bf16 with fp32 q, out and cache (the reference without
+ * autocast; head_dim a multiple of 4, no alignment beyond the elements'); the
+ * out rows t >= new_lens[b] are written as zeros. */
+int tt_prefill_attn_f32(const void *q, const int64_t q_strides[3],
+                        const void *k_cache, const void *v_cache, const int64_t cache_strides[3],
+                        const int32_t *positions, const int32_t *new_lens, int64_t max_seq_len,
+                        const int32_t *page_table, int64_t max_pages, int64_t num_pages,
+                        void *out, const int64_t out_strides[3],
+                        int64_t batch, int64_t num_new, int64_t num_q_heads, int64_t num_kv_heads,
+                        int64_t head_dim, int64_t page_size, float sm_scale, tt_stream_t stream);
+
 /* As tt_prefill_attn_bf16 with an fp8-e4m3fn cache and per-(token, head) scales. */
 int tt_prefill_attn_fp8(const void *q, const int64_t q_strides[3],
                         const void *k_cache, const void *v_cache,

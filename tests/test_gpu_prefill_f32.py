@@ -1,0 +1,81 @@
+"""GPU parity: fp32 prefill attention (tt_prefill_attn_f32) vs the fp64 oracle
+and vs row attention, at the edges of its tiles: head dims filling and padding
+each tile width, chunks that end inside, at and after a 32-key tile and a
+wave's turn, one and two column blocks per workgroup, group sizes that leave
+columns idle, rows past new_lens (zeros), NaN in every unused slot.
+
+Tolerance as for the row attention tests' fp32 caches: 1e-5 + 1e-4 |ref| (fp32
+operands and sums of up to 1300 terms in another order).
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle.attention import prefill_attention as ref_prefill
+from tests.kv_inputs import sm_scale
+from tests.test_gpu_rows_attention import _cache, _dev, _queries
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(cached, new, Hq, Hkv, D, paged, seed=0, T=None, edit=None):
+    from tinytron_amd import ops
+
+    rng = np.random.default_rng(seed)
+    T = T or max(new)
+    kv, keys, values = _cache([c + n for c, n in zip(cached, new)], Hkv, D, "f32", paged, rng)
+    if edit is not None:
+        edit(kv, values)
+    q, qf = _queries(rng, (len(cached), Hq, T, D), "f32")
+    assert ops.prefill_f32_supported(kv, Hq)
+    pos = torch.tensor(cached, dtype=torch.int32, device="cuda")
+    nl = torch.tensor(new, dtype=torch.int32, device="cuda")
+    out = torch.full((len(cached), T, Hq, D), float("nan"), device="cuda")
+    ops.prefill_attention_f32(q, kv, pos, max(c + n for c, n in zip(cached, new)), new_lens=nl, out=out)
+    torch.cuda.synchronize()
+    ref = ref_prefill(qf, keys, values, cached, new, Hkv, sm_scale(D))
+    return out.cpu().numpy(), ref, (ops, q, kv)
+
+
+def _check(got, ref, new):
+    for b, n in enumerate(new):
+        assert np.all(got[b, n:] == 0.0)
+        err = np.abs(got[b, :n] - ref[b][:n])
+        assert np.all(err <= 1e-5 + 1e-4 * np.abs(ref[b][:n])), (b, float(err.max()))
+
+
+@pytest.mark.parametrize("D", [4, 20, 32, 36, 64, 96, 128])
+@pytest.mark.parametrize("paged", [False, True])
+def test_head_dims(D, paged):
+    cached, new = [0, 40, 5, 127, 0], [33, 1, 17, 66, 0]
+    got, ref, _ = _run(cached, new, 6, 2, D, paged, seed=D)
+    _check(got, ref, new)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(4, 4), (5, 1), (16, 1), (16, 8)])
+def test_groups_and_long_prefix(Hq, Hkv):
+    # past one 1024-token page-entry span; keys at 31, 32, 33 and 127 .. 129
+    cached, new = [1250, 30, 0], [37, 3, 129]
+    got, ref, _ = _run(cached, new, Hq, Hkv, 64, True, seed=Hq)
+    _check(got, ref, new)
+
+
+def test_two_blocks_per_workgroup():
+    # 8 sequences x 8 heads x 130 / 8 token blocks: past two workgroups per CU
+    cached, new = [0, 3, 64, 0, 1, 0, 31, 2], [130, 64, 9, 17, 130, 1, 100, 16]
+    got, ref, (ops, q, kv) = _run(cached, new, 32, 8, 32, False, seed=9)
+    _check(got, ref, new)
+    rows = ops.prefill_attention_rows(q, kv, cached, new)
+    assert torch.allclose(torch.from_numpy(got), rows.cpu(), rtol=1e-4, atol=1e-5)
+
+
+def test_infinite_value_of_a_later_token_stays_there():
+    # value row 20 is inf: token 20 and later see it, earlier ones (same tile) must not
+    def edit(kv, values):
+        off = 20 * 64
+        kv.v[off:off + 64] = float("inf")
+
+    got, ref, _ = _run([0], [40], 4, 1, 64, False, seed=3, edit=edit)
+    _check(got[:, :20], [r[:20] for r in ref], [20])
+    assert np.all(np.isinf(got[0, 20:]))

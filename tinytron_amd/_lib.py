@@ -133,6 +133,7 @@ SIGNATURES = {
     "tt_decode_pick_split": ([_vp, _i64, _i64, _i64, ctypes.c_int32], ctypes.c_int64),
     "tt_decode_workspace_bytes": ([_i64, _i64, _i64, _i64, _i64, _i64], ctypes.c_size_t),
     "tt_prefill_attn_bf16": ([_vp, _i64p, _vp, _vp, _i64p] + _PREFILL_TAIL, ctypes.c_int),
+    "tt_prefill_attn_f32": ([_vp, _i64p, _vp, _vp, _i64p] + _PREFILL_TAIL, ctypes.c_int),
     "tt_prefill_attn_fp8": ([_vp, _i64p, _vp, _vp, _vp, _vp, _i64p] + _PREFILL_TAIL, ctypes.c_int),
     "tt_linear_splitk_bf16": ([_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp], ctypes.c_int),
     "tt_linear_splitk_packed_bf16": ([_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp], ctypes.c_int),

@@ -256,9 +256,10 @@ class _LayerCacheBase:
         [B, H_q, T, D], new_lens[b] tokens of sequence b) over each sequence's
         cache; returns [B, T, H_q, D]. bf16 activations over a bf16 / fp8 cache
         whose rows are whole 16-byte fragments take the prefill kernel (rows
-        past new_lens[b] untouched); fp32 and the other head dims take row
-        attention, one query row per new token (rows past new_lens[b] zero;
-        ``kernel=False`` takes it for every case)."""
+        past new_lens[b] untouched), fp32 over such an fp32 cache its fp32
+        counterpart; the other head dims take row attention, one query row per
+        new token (``kernel=False`` takes it for every case). fp32 and row
+        attention leave zeros in the rows past new_lens[b]."""
         lay = self.layout
         T = q_rot.shape[2]
         if kernel and q_rot.dtype == torch.bfloat16 and lay.kind in ("bf16", "fp8") \
@@ -268,6 +269,10 @@ class _LayerCacheBase:
             nl = torch.tensor([int(n) for n in new_lens], dtype=torch.int32).to(prev.device, non_blocking=True)
             return ops.prefill_attention(q_rot, lay, prev, self.current_length, new_lens=nl, out=out)
         adds = [min(int(n), T) for n in new_lens]
+        if kernel and q_rot.dtype == torch.float32 and ops.prefill_f32_supported(lay, q_rot.shape[1]):
+            prev = self._lens_dev[1 - self._cur]
+            nl = torch.tensor(adds, dtype=torch.int32).to(prev.device, non_blocking=True)
+            return ops.prefill_attention_f32(q_rot, lay, prev, self.current_length, new_lens=nl, out=out)
         cached = [x - a for x, a in zip(self._host_lens, adds)]
         if self.workspace is None:
             self.workspace = ops.Workspace(q_rot.device)

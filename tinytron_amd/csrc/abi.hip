@@ -498,8 +498,10 @@ int prefill_common(tt::CacheKind kind, const void *q, const int64_t q_strides[3]
            "num_attention_heads must be divisible by num_key_value_heads");
   const int64_t g = num_q_heads / num_kv_heads;
   TT_CHECK(g <= 16, TT_ERR_UNSUPPORTED, "GQA group size %lld > 16 is not supported", (long long)g);
-  TT_CHECK(tt::tile_head_dim(head_dim, kind) > 0, TT_ERR_UNSUPPORTED,
-           "prefill attention needs head_dim <= 128 and a multiple of 8 (bf16 cache) or 16 (fp8 cache), got %lld",
+  const bool f32 = kind == tt::CacheKind::kF32;
+  TT_CHECK(f32 ? tt::prefill_f32_supported(head_dim) : tt::tile_head_dim(head_dim, kind) > 0, TT_ERR_UNSUPPORTED,
+           "prefill attention needs head_dim <= 128 and a multiple of 4 (fp32 cache), 8 (bf16 cache) or 16 (fp8 "
+           "cache), got %lld",
            (long long)head_dim);
   TT_CHECK(max_seq_len >= 0 && max_seq_len < ((int64_t)1 << 30), TT_ERR_INVALID_ARGUMENT, "max_seq_len out of range");
   TT_CHECK(batch * num_kv_heads < ((int64_t)1 << 26) && num_new < ((int64_t)1 << 24), TT_ERR_UNSUPPORTED,
@@ -526,12 +528,14 @@ int prefill_common(tt::CacheKind kind, const void *q, const int64_t q_strides[3]
     rc = check_contiguous_room(max_seq_len, head_dim, cache_strides, batch, num_kv_heads);
     if (rc != TT_OK) return rc;
   }
-  TT_CHECK(aligned(q, 16) && aligned(k_cache, 16) && aligned(v_cache, 16), TT_ERR_INVALID_ARGUMENT,
-           "q and cache pointers must be 16-byte aligned");
-  TT_CHECK(q_strides[0] % 8 == 0 && q_strides[1] % 8 == 0 && q_strides[2] % 8 == 0, TT_ERR_INVALID_ARGUMENT,
-           "q strides must be multiples of 8 elements");
-  TT_CHECK(cache_strides[0] % 8 == 0 && cache_strides[1] % 8 == 0 && cache_strides[2] % 8 == 0,
-           TT_ERR_INVALID_ARGUMENT, "cache strides must be multiples of 8 elements");
+  if (!f32) {
+    TT_CHECK(aligned(q, 16) && aligned(k_cache, 16) && aligned(v_cache, 16), TT_ERR_INVALID_ARGUMENT,
+             "q and cache pointers must be 16-byte aligned");
+    TT_CHECK(q_strides[0] % 8 == 0 && q_strides[1] % 8 == 0 && q_strides[2] % 8 == 0, TT_ERR_INVALID_ARGUMENT,
+             "q strides must be multiples of 8 elements");
+    TT_CHECK(cache_strides[0] % 8 == 0 && cache_strides[1] % 8 == 0 && cache_strides[2] % 8 == 0,
+             TT_ERR_INVALID_ARGUMENT, "cache strides must be multiples of 8 elements");
+  }
   if (batch == 0 || num_new == 0) return ok();
 
   tt::PrefillArgs a{};
@@ -566,10 +570,9 @@ int prefill_common(tt::CacheKind kind, const void *q, const int64_t q_strides[3]
   a.positions = positions;
   a.new_lens = new_lens;
   a.num_new = (int)num_new;
-  a.qt = (int)(16 / g);
-  a.nq = (int)((num_new + a.qt - 1) / a.qt);
-  a.wg_per_pair = (a.nq + tt::kWavesPerBlock - 1) / tt::kWavesPerBlock;
   (void)hipGetLastError();
+  if (f32)
+    return from_hip(tt::launch_prefill_attn_f32(a, (int)head_dim, (hipStream_t)stream), "prefill attention launch");
   return from_hip(tt::launch_prefill_attn(a, kind, (int)head_dim, (hipStream_t)stream), "prefill attention launch");
 }
 
@@ -731,6 +734,17 @@ int tt_prefill_attn_bf16(const void *q, const int64_t q_strides[3], const void *
                          int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
                          float sm_scale, tt_stream_t stream) {
   return prefill_common(tt::CacheKind::kBF16, q, q_strides, k_cache, v_cache, nullptr, nullptr, cache_strides,
+                        positions, new_lens, max_seq_len, page_table, max_pages, num_pages, out, out_strides, batch,
+                        num_new, num_q_heads, num_kv_heads, head_dim, page_size, sm_scale, stream);
+}
+
+int tt_prefill_attn_f32(const void *q, const int64_t q_strides[3], const void *k_cache, const void *v_cache,
+                        const int64_t cache_strides[3], const int32_t *positions, const int32_t *new_lens,
+                        int64_t max_seq_len, const int32_t *page_table, int64_t max_pages, int64_t num_pages,
+                        void *out, const int64_t out_strides[3], int64_t batch, int64_t num_new,
+                        int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
+                        float sm_scale, tt_stream_t stream) {
+  return prefill_common(tt::CacheKind::kF32, q, q_strides, k_cache, v_cache, nullptr, nullptr, cache_strides,
                         positions, new_lens, max_seq_len, page_table, max_pages, num_pages, out, out_strides, batch,
                         num_new, num_q_heads, num_kv_heads, head_dim, page_size, sm_scale, stream);
 }

@@ -180,13 +180,15 @@ struct PrefillArgs : DecodeArgs {
   const int32_t *positions;    // [B] tokens cached before the new ones
   const int32_t *new_lens;     // [B] new tokens per sequence (<= num_new), or null for all num_new
   int num_new;                 // T
-  int qt;                      // query tokens per wave (16 / G)
-  int nq;                      // query blocks per sequence: ceil(T / qt)
-  int wg_per_pair;             // workgroups per (sequence, KV head): ceil(nq / 4)
+  int qt;                      // query tokens per block of columns (set by the launcher)
+  int wg_per_pair;             // workgroups per (sequence, KV head) (set by the launcher)
   int vec_out;                 // out 8-byte aligned, strides multiples of 4: 4 head_dim entries per store
 };
 
 hipError_t launch_prefill_attn(const PrefillArgs &a, CacheKind kind, int head_dim, hipStream_t stream);
+// fp32 caches: whole 16-byte fragments (head_dim a multiple of 4, <= 128); rows past new_lens are zeroed
+bool prefill_f32_supported(int64_t head_dim);
+hipError_t launch_prefill_attn_f32(const PrefillArgs &a, int head_dim, hipStream_t stream);
 
 // Token sampling: one workgroup per row of logits [M, V] (bf16 or fp32).
 struct SampleArgs {

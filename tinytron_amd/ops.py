@@ -764,10 +764,34 @@ def prefill_attention(q: torch.Tensor, layout: KVLayout, positions: torch.Tensor
     [B] (optional) = new tokens per sequence; returns out [B, T, H_q, D]
     (rows t >= new_lens[b] untouched). Restates the prefill branch of the
     reference attention (attn.py:321-341) for a ragged batch."""
+    if q.dtype != torch.bfloat16 or layout.kind not in ("bf16", "fp8"):
+        _require_cuda(q, layout.k, layout.v, positions)
+        raise ValueError("prefill_attention takes bf16 q with a bf16 or fp8 cache")
+    return _prefill_attention(q, layout, positions, max_seq_len, new_lens, out, sm_scale)
+
+
+def prefill_f32_supported(layout: KVLayout, num_q_heads: int) -> bool:
+    """Whether prefill_attention_f32 takes this cache: fp32 rows that are whole
+    16-byte fragments (head_dim a multiple of 4, at most 128), groups of at
+    most 16 query heads and, in the contiguous store, dense pages."""
+    return (layout.kind == "f32" and layout.head_dim % 4 == 0 and layout.head_dim <= 128
+            and num_q_heads % layout.num_heads == 0 and num_q_heads // layout.num_heads <= 16
+            and (layout.page_table is not None or layout.strides[1] == layout.page_size * layout.head_dim))
+
+
+def prefill_attention_f32(q: torch.Tensor, layout: KVLayout, positions: torch.Tensor, max_seq_len: int,
+                          new_lens: torch.Tensor | None = None, out: torch.Tensor | None = None,
+                          sm_scale: float | None = None) -> torch.Tensor:
+    """prefill_attention for fp32 activations over an fp32 cache (the reference
+    without autocast, attn.py:321-341); rows t >= new_lens[b] are zeros."""
+    if q.dtype != torch.float32 or layout.kind != "f32":
+        raise ValueError("prefill_attention_f32 takes fp32 q with an fp32 cache")
+    return _prefill_attention(q, layout, positions, max_seq_len, new_lens, out, sm_scale)
+
+
+def _prefill_attention(q, layout, positions, max_seq_len, new_lens, out, sm_scale):
     _require_cuda(q, layout.k, layout.v, positions)
     _check_lastdim("q", q, 4)
-    if q.dtype != torch.bfloat16 or layout.kind not in ("bf16", "fp8"):
-        raise ValueError("prefill_attention takes bf16 q with a bf16 or fp8 cache")
     B, Hq, T, D = q.shape
     if D != layout.head_dim:
         raise ValueError(f"head_dim {D} does not match the cache's {layout.head_dim}")
@@ -778,7 +802,7 @@ def prefill_attention(q: torch.Tensor, layout: KVLayout, positions: torch.Tensor
     if max_seq_len > layout.capacity:
         raise ValueError(f"max_seq_len {max_seq_len} exceeds the cache capacity {layout.capacity}")
     if out is None:
-        out = torch.empty(B, T, Hq, D, dtype=torch.bfloat16, device=q.device)
+        out = torch.empty(B, T, Hq, D, dtype=q.dtype, device=q.device)
     _check_lastdim("out", out, 4)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D)
@@ -790,8 +814,10 @@ def prefill_attention(q: torch.Tensor, layout: KVLayout, positions: torch.Tensor
             float(sm_scale), _stream(q.device)]
     if layout.kind == "fp8":
         st = lib.tt_prefill_attn_fp8(*head, _ptr(layout.k_scale), _ptr(layout.v_scale), *tail)
-    else:
+    elif layout.kind == "bf16":
         st = lib.tt_prefill_attn_bf16(*head, *tail)
+    else:
+        st = lib.tt_prefill_attn_f32(*head, *tail)
     _lib.check(st, "prefill_attention")
     return out
 
