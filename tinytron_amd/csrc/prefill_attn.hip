@@ -172,7 +172,7 @@ __device__ __forceinline__ void stage_store(const DecodeArgs &a, const Staged<D,
 // Lazy running maximum: a column's reference moves only when a tile's maximum
 // exceeds it by more than kLazyMax (log2 units), so P <= 2^kLazyMax (fp32 O and
 // l and the bf16 P halves have the range) and most tiles need no rescale.
-constexpr float kLazyMax = 8.0f;
+constexpr float kLazyMax = 7.0f;
 
 // p (one lane's 8 softmax values of a contraction step) as bf16 P_hi + P_lo:
 // P_lo = bf16(p - P_hi), the difference exact in fp32.
@@ -358,9 +358,9 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
           bf16x8 hi, lo;
           split_p(p, hi, lo);
 #pragma unroll
-          for (int c = 0; c < D / 32; ++c) o[c] = mfma32(vf[c], hi, o[c]);
+          for (int c = 0; c < D / 32; ++c) o[c] = mfma32(vf[c], lo, o[c]);  // the small terms first
 #pragma unroll
-          for (int c = 0; c < D / 32; ++c) o[c] = mfma32(vf[c], lo, o[c]);
+          for (int c = 0; c < D / 32; ++c) o[c] = mfma32(vf[c], hi, o[c]);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
