@@ -577,7 +577,7 @@ size_t tt_decode_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t num
  * 44-45); the rows of several projections of one input may be stacked into
  * one weight (q|k|v, gate|up). x bf16 [M, K] (row stride ldx), weight bf16
  * [N, K] (row stride ldw). Requirements: N % 64 == 0, K % k_chunk == 0,
- * k_chunk in {256, 512, 1024}, 16-byte aligned pointers, strides multiples
+ * k_chunk in {256, 512, 1024}, or 1280 for m <= 32, 16-byte aligned pointers, strides multiples
  * of 8.
  */
 int tt_linear_splitk_bf16(const void *x, int64_t ldx, const void *weight, int64_t ldw, float *partials, int64_t m,

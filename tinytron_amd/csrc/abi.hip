@@ -461,8 +461,9 @@ int linear_common(const void *x, int64_t ldx, const void *weight, int64_t ldw, i
                   int64_t m, int64_t n, int64_t k, int64_t k_chunk, tt_stream_t stream) {
   TT_CHECK(x && weight && partials, TT_ERR_INVALID_ARGUMENT, "a required pointer is NULL");
   TT_CHECK(m >= 0 && m <= 65535 * 64 && n > 0 && k > 0, TT_ERR_INVALID_ARGUMENT, "bad GEMM shape");
-  TT_CHECK(k_chunk == 256 || k_chunk == 512 || k_chunk == 1024, TT_ERR_INVALID_ARGUMENT,
-           "k_chunk must be 256, 512 or 1024, got %lld", (long long)k_chunk);
+  TT_CHECK(k_chunk == 256 || k_chunk == 512 || k_chunk == 1024 || (k_chunk == 1280 && m <= 32),
+           TT_ERR_INVALID_ARGUMENT, "k_chunk must be 256, 512 or 1024 (for up to 32 rows also 1280), got %lld",
+           (long long)k_chunk);
   TT_CHECK(n % 64 == 0 && k % k_chunk == 0, TT_ERR_UNSUPPORTED,
            "N must be a multiple of 64 and K of k_chunk (N %lld, K %lld, k_chunk %lld)", (long long)n, (long long)k,
            (long long)k_chunk);

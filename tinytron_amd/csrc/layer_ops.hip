@@ -49,34 +49,43 @@ __device__ __forceinline__ const uint16_t *wfrag_base(const SkinnyGemmArgs &a, i
   return a.w + (int64_t)(nb * 16 + (lane & 15)) * a.ldw + k + 8 * (lane >> 4);
 }
 
-// Workgroups of this shape meant to share a CU (bounded by the x chunk's LDS
-// footprint, 64 x (KC + 8) x 2 bytes), and the waves per SIMD the register
-// allocation must leave room for so that they can.
+// Waves per SIMD the register allocation must leave room for. 64-row tiles
+// (MB = 4): the workgroups of this shape meant to share a CU, bounded by the x
+// chunk's LDS footprint (64 x (KC + 8) x 2 bytes). Narrower tiles: what the
+// weight burst's registers (KC / 8 per lane) allow.
 constexpr int gemm_wgs_per_cu(int kc, int waves) {
   return kc == 256 ? (waves <= 4 ? 4 : waves <= 8 ? 2 : 1) : kc == 512 ? (waves <= 8 ? 2 : 1) : 1;
 }
 
-template <int KC, int WAVES>
+template <int KC, int WAVES, int MB>
 constexpr int gemm_min_waves() {
+  if (MB < 4) return KC <= 512 ? 4 : 2;
   const int w = (WAVES * gemm_wgs_per_cu(KC, WAVES) + 3) / 4;
   return w < 1 ? 1 : w > 4 ? 4 : w;
 }
 
-template <int KC, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, (gemm_min_waves<KC, WAVES>())) void skinny_gemm_kernel(SkinnyGemmArgs a) {
+// MB: 16-row blocks of x per workgroup (rows past M are zero). M <= 16 and <= 32
+// take MB = 1 and 2: a quarter or half of the LDS, its staging loads and MFMAs,
+// so that more workgroups stream weights on each CU. At M = 5, weights cold (us,
+// 64-row tiles -> 16-row): N 2048, K 6144 (512-wide chunks) 7.6 -> 6.6; N 5120,
+// K 5120 12.0 -> 10.8; N 27648, K 5120 55.7 -> 54.4, 1024-wide 81.4 -> 54.7
+// (one 64-row workgroup per CU there). M = 17 .. 32 at 1024-wide chunks: N 27648
+// 84.9 -> 74.5.
+template <int KC, int WAVES, int MB>
+__global__ __launch_bounds__(64 * WAVES, (gemm_min_waves<KC, WAVES, MB>())) void skinny_gemm_kernel(SkinnyGemmArgs a) {
   constexpr int KSTEPS = KC / 32;
   constexpr int ROW = KC + 8;  // padded LDS row (elements): 16 consecutive rows hit distinct banks
-  __shared__ __attribute__((aligned(16))) uint16_t xs[64 * ROW];
+  __shared__ __attribute__((aligned(16))) uint16_t xs[16 * MB * ROW];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int n0 = blockIdx.x * (16 * WAVES) + wave * 16;
   const int64_t k0 = (int64_t)blockIdx.y * KC;
-  const int m0 = blockIdx.z * 64;
+  const int m0 = blockIdx.z * (16 * MB);
 
-  // x rows m0 .. m0 + 63 of the chunk (L2-resident, rows past M are zero)
+  // the tile's x rows of the chunk (L2-resident, rows past M are zero)
   // are loaded before the weights: vector loads return in issue order, so
   // x issued first can go to LDS while the weight stream is still in flight.
-  constexpr int XN = 64 * (KC / 8);                        // 16-byte pieces of the x chunk
+  constexpr int XN = 16 * MB * (KC / 8);                   // 16-byte pieces of the x chunk
   constexpr int XL = (XN + 64 * WAVES - 1) / (64 * WAVES);  // per thread
   u32x4 xr[XL];
 #pragma unroll
@@ -106,14 +115,14 @@ __global__ __launch_bounds__(64 * WAVES, (gemm_min_waves<KC, WAVES>())) void ski
   }
   __syncthreads();
 
-  f32x4 acc[4];
+  f32x4 acc[MB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
     const bf16x8 af = __builtin_bit_cast(bf16x8, wf[s]);
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
+    for (int mb = 0; mb < MB; ++mb) {
       const bf16x8 bfr =
           *reinterpret_cast<const bf16x8 *>(xs + (mb * 16 + (lane & 15)) * ROW + 32 * s + 8 * (lane >> 4));
       acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr, acc[mb], 0, 0, 0);
@@ -123,7 +132,7 @@ __global__ __launch_bounds__(64 * WAVES, (gemm_min_waves<KC, WAVES>())) void ski
   // acc[mb]: lane (j + 16g) holds out column n0 + 4g + r (r = 0..3) of batch row m0 + 16 mb + j.
   float *P = a.part + (int64_t)blockIdx.y * a.M * a.N;
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
+  for (int mb = 0; mb < MB; ++mb) {
     const int m = m0 + mb * 16 + (lane & 15);
     if (m < a.M) *reinterpret_cast<f32x4 *>(P + (int64_t)m * a.N + n0 + 4 * (lane >> 4)) = acc[mb];
   }
@@ -172,11 +181,14 @@ __global__ __launch_bounds__(256) void reduce_bf16_kernel(const float *P, int S,
   *reinterpret_cast<uint2 *>(y + i) = make_uint2(lo, hi);
 }
 
-__device__ __forceinline__ float block_sum_256(float v, float *red) {
+template <int kThreads>
+__device__ __forceinline__ float block_sum(float v, float *red) {
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  const float t = red[0] + red[1] + red[2] + red[3];
+  float t = red[0];
+#pragma unroll
+  for (int w = 1; w < kThreads / 64; ++w) t += red[w];
   __syncthreads();
   return t;
 }
@@ -187,20 +199,23 @@ __device__ __forceinline__ float block_sum_256(float v, float *red) {
 // the first add, so the row costs one memory round trip; the splits are added
 // in order. (Loaded after the block reduction, the weight cost two more round
 // trips: the compiler keeps loads below a barrier where the source puts them.)
-// PER float4 groups per thread (C <= 1024 * PER, C a multiple of 4; with
+// PER float4 groups per thread (C <= 4 * kThreads * PER, C a multiple of 4; with
 // kMask, groups past C are neither loaded nor stored and add 0 to the sum of
-// squares; without it C == 1024 * PER and every load is unconditional, so
+// squares; without it C == 4 * kThreads * PER and every load is unconditional, so
 // all of them go out before the first add); SMAX splits loaded at once
-template <int PER, int SMAX, bool kMask>
-__global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *x, const float *P, int S, int64_t MN,
+// (kThreads = 1024: rows wider than 2048 with many splits, where 256 threads
+// walk the splits four at a time, a memory round trip each: the norms of 5 rows
+// of 5120 after 10 and 27 splits, 24 us; in batches of 8 by 1024 threads, ~4)
+template <int PER, int SMAX, bool kMask, int kThreads>
+__global__ __launch_bounds__(kThreads) void add_rmsnorm_kernel(float *x, const float *P, int S, int64_t MN,
                                                           const float *w, float eps, uint16_t *y, int C) {
-  __shared__ float red[4];
+  __shared__ float red[kThreads / 64];
   const int64_t row = (int64_t)blockIdx.x * C;
   f32x4 v[PER], wv[PER];
   f32x4 pv[PER][SMAX];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int c = 4 * (threadIdx.x + 256 * j);
+    const int c = 4 * (threadIdx.x + kThreads * j);
     const bool in = !kMask || c < C;
     v[j] = in ? *reinterpret_cast<const f32x4 *>(x + row + c) : f32x4{0.f, 0.f, 0.f, 0.f};
     if (P != nullptr) {
@@ -212,20 +227,32 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *x, const float 
   }
 #pragma unroll
   for (int j = 0; j < PER; ++j) {  // issued after the row's loads, which are needed first
-    const int c = 4 * (threadIdx.x + 256 * j);
+    const int c = 4 * (threadIdx.x + kThreads * j);
     wv[j] = !kMask || c < C ? *reinterpret_cast<const f32x4 *>(w + c) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int c = 4 * (threadIdx.x + 256 * j);
+    const int c = 4 * (threadIdx.x + kThreads * j);
     if (kMask && c >= C) continue;
     if (P != nullptr) {
       f32x4 d = pv[j][0];
 #pragma unroll
       for (int s = 1; s < SMAX; ++s)
         if (s < S) d += pv[j][s];
-      for (int s = SMAX; s < S; ++s) d += *reinterpret_cast<const f32x4 *>(P + (int64_t)s * MN + row + c);
+      if constexpr (kThreads == 256) {  // S <= SMAX but for C <= 2048 and more than 16 splits
+        for (int s = SMAX; s < S; ++s) d += *reinterpret_cast<const f32x4 *>(P + (int64_t)s * MN + row + c);
+      } else {
+        for (int s0 = SMAX; s0 < S; s0 += SMAX) {  // further batches of SMAX splits, a round trip each
+          f32x4 more[SMAX];
+#pragma unroll
+          for (int s = 0; s < SMAX; ++s)
+            more[s] = *reinterpret_cast<const f32x4 *>(P + (int64_t)(s0 + s < S ? s0 + s : 0) * MN + row + c);
+#pragma unroll
+          for (int s = 0; s < SMAX; ++s)
+            if (s0 + s < S) d += more[s];
+        }
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[j][e] += round_bf16(d[e]);
       *reinterpret_cast<f32x4 *>(x + row + c) = v[j];
@@ -233,11 +260,11 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *x, const float 
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
   }
-  const float var = block_sum_256(ss, red) / (float)C;
+  const float var = block_sum<kThreads>(ss, red) / (float)C;
   const float r = 1.0f / sqrtf(var + eps);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int c = 4 * (threadIdx.x + 256 * j);
+    const int c = 4 * (threadIdx.x + kThreads * j);
     if (kMask && c >= C) continue;
     uint32_t lo = pack_bf16x2(wv[j][0] * (v[j][0] * r), wv[j][1] * (v[j][1] * r));
     uint32_t hi = pack_bf16x2(wv[j][2] * (v[j][2] * r), wv[j][3] * (v[j][3] * r));
@@ -298,7 +325,10 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float *P, int S, in
 // that divides I / 8: 3 where it can, the measured layout).
 // (Register budget: two workgroups' worth per CU, as measured for NB = 3;
 // NB = 4 with 128 weight registers per lane fits one.)
-template <int K, int NB>
+// MB 16-row blocks of x per workgroup, as the split-K GEMM: with MB <= 2 every
+// round's x fits the LDS, so all of it is staged before the weights and no round
+// waits for the one before (K 2048, I 6144, M = 5: 14.4 -> 10.3 us; M = 32 12.0; K 1024, I 4096: 6.6 -> 5.3).
+template <int K, int NB, int MB>
 __global__ __launch_bounds__(64 * 2 * NB, NB == 4 ? 1 : 2) void swiglu_gemm_kernel(SwigluGemmArgs a) {
   constexpr int R = (K + 1023) / 1024; // staging rounds
   constexpr int KS = K / 64;           // k steps per wave (its half of K)
@@ -306,30 +336,36 @@ __global__ __launch_bounds__(64 * 2 * NB, NB == 4 ? 1 : 2) void swiglu_gemm_kern
   constexpr int ROW = 512 + 8;         // padded LDS row (elements): one 1 KiB DMA chunk
   static_assert((K == 768 || K == 1024 || K == 2048) && KQ <= 512 && KS <= 32, "K = 768, 1024 or 2048");
   constexpr int kWaves = 2 * NB;
-  constexpr int kRows = 2 * 64;        // LDS rows per round: 2 halves x 64 x rows
-  __shared__ __attribute__((aligned(16))) uint16_t xs[kRows * ROW];
+  constexpr int kM = 16 * MB;          // x rows of the tile
+  constexpr int kRows = 2 * kM;        // LDS rows per round: 2 halves x the x rows
+  constexpr int kBufs = MB <= 2 ? R : 1;
+  constexpr int kRed = 2 * NB * ((MB + 1) / 2) * 64 * 16;  // bytes of the halves' exchange
+  constexpr int kXs = kBufs * kRows * ROW * 2;
+  __shared__ __attribute__((aligned(16))) uint16_t xs[(kXs > kRed ? kXs : kRed) / 2];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int blk = wave >> 1;           // row block of this workgroup
   const int half = wave & 1;           // K half
   const int nb = blockIdx.x * NB + blk;
-  const int m0 = blockIdx.z * 64;
-  const int mrows = min(64, a.M - m0);
+  const int m0 = blockIdx.z * kM;
+  const int mrows = min(kM, a.M - m0);
 
   // x rows m0 .. m0 + mrows - 1; offsets past the last valid row's data read zero
   const auto rx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t *>(a.x) + (int64_t)m0 * a.ldx, (short)0,
       (int)(((int64_t)(mrows - 1) * a.ldx + K) * 2), 0x00020000);
   auto stage = [&](int round) {
-    for (int i = wave; i < kRows; i += kWaves) {  // i = h * 64 + row
-      const int h = i >> 6, r = i & 63;
+    uint16_t *buf = xs + (kBufs > 1 ? round : 0) * kRows * ROW;
+    for (int i = wave; i < kRows; i += kWaves) {  // i = h * kM + row
+      const int h = i / kM, r = i % kM;
       const int col = h * (K / 2) + round * KQ;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void *)(xs + i * ROW), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void *)(buf + i * ROW), 16,
                                                16 * lane + (int)(((int64_t)r * a.ldx + col) * 2), 0, 0, 0);
     }
   };
 
-  stage(0);
+#pragma unroll
+  for (int round = 0; round < kBufs; ++round) stage(round);
   __builtin_amdgcn_sched_barrier(0);
   const uint16_t *wrow = a.w + (((int64_t)nb * (K / 32) + half * KS) * 64 + lane) * 8;
   u32x4 wf[KS];
@@ -341,13 +377,14 @@ __global__ __launch_bounds__(64 * 2 * NB, NB == 4 ? 1 : 2) void swiglu_gemm_kern
   __builtin_amdgcn_s_waitcnt((KS & 15) | (7 << 4) | (15 << 8) | (((KS >> 4) & 3) << 14));  // this wave's x DMA
   __syncthreads();
 
-  f32x4 acc[4];
+  f32x4 acc[MB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint16_t *xrow = xs + (half * 64 + (lane & 15)) * ROW + 8 * (lane >> 4);
+  for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint16_t *xrow0 = xs + (half * kM + (lane & 15)) * ROW + 8 * (lane >> 4);
 #pragma unroll
   for (int round = 0; round < R; ++round) {
-    if (round > 0) {
+    const uint16_t *xrow = xrow0 + (kBufs > 1 ? round : 0) * kRows * ROW;
+    if (kBufs == 1 && round > 0) {
       __syncthreads();  // every wave is done with the previous round's x
       stage(round);
       __builtin_amdgcn_s_waitcnt((0 & 15) | (7 << 4) | (15 << 8));
@@ -357,24 +394,29 @@ __global__ __launch_bounds__(64 * 2 * NB, NB == 4 ? 1 : 2) void swiglu_gemm_kern
     for (int s = 0; s < KS / R; ++s) {
       const bf16x8 af = __builtin_bit_cast(bf16x8, wf[round * (KS / R) + s]);
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
+      for (int mb = 0; mb < MB; ++mb) {
         const bf16x8 bfr = *reinterpret_cast<const bf16x8 *>(xrow + mb * 16 * ROW + 32 * s);
         acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfr, acc[mb], 0, 0, 0);
       }
     }
   }
 
-  // the halves meet: half 0 finishes m blocks 0-1, half 1 blocks 2-3
+  // the halves meet: half 0 finishes the first (MB + 1) / 2 m blocks, half 1
+  // the rest (register indices stay constants: each half has its own branch)
+  constexpr int kFirst = (MB + 1) / 2;
   __syncthreads();
-  f32x4 *red = reinterpret_cast<f32x4 *>(xs);  // [block][half][2][64]
+  f32x4 *red = reinterpret_cast<f32x4 *>(xs);  // [block][half][kFirst][64]
+  f32x4 *send = red + (blk * 2 + half) * kFirst * 64 + lane;
+  if (half == 0) {  // uniform
 #pragma unroll
-  for (int j = 0; j < 2; ++j) red[((blk * 2 + half) * 2 + j) * 64 + lane] = acc[half == 0 ? 2 + j : j];
+    for (int j = kFirst; j < MB; ++j) send[(j - kFirst) * 64] = acc[j];
+  } else {
+#pragma unroll
+    for (int j = 0; j < kFirst; ++j) send[j * 64] = acc[j];
+  }
   __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int mb = half == 0 ? j : 2 + j;
-    const f32x4 other = red[((blk * 2 + (1 - half)) * 2 + j) * 64 + lane];
-    const f32x4 sum = half == 0 ? acc[mb] + other : other + acc[mb];
+  const f32x4 *recv = red + (blk * 2 + (1 - half)) * kFirst * 64 + lane;
+  auto finish = [&](int mb, f32x4 sum) {
     f32x4 up;
 #pragma unroll
     for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(sum[r], 32, 64);
@@ -386,6 +428,13 @@ __global__ __launch_bounds__(64 * 2 * NB, NB == 4 ? 1 : 2) void swiglu_gemm_kern
       *reinterpret_cast<uint2 *>(a.out + (int64_t)(m0 + row) * a.ldo + 8 * nb + 4 * (lane >> 4)) =
           make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
     }
+  };
+  if (half == 0) {
+#pragma unroll
+    for (int j = 0; j < kFirst; ++j) finish(j, acc[j] + recv[j * 64]);
+  } else {
+#pragma unroll
+    for (int j = kFirst; j < MB; ++j) finish(j, recv[(j - kFirst) * 64] + acc[j]);
   }
 }
 
@@ -427,7 +476,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_rows_kernel(float *x, const u
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
   }
-  const float var = block_sum_256(ss, red) / (float)C;
+  const float var = block_sum<256>(ss, red) / (float)C;
   const float r = 1.0f / sqrtf(var + eps);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -465,11 +514,31 @@ __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const uint16_t *g_in
 
 }  // namespace
 
+template <int KC, int MB>
+hipError_t launch_gemm_tile(const SkinnyGemmArgs &a, int waves, hipStream_t stream) {
+  const dim3 grid((unsigned)(a.N / (16 * waves)), (unsigned)(a.K / KC), (unsigned)((a.M + 16 * MB - 1) / (16 * MB)));
+  if (waves == 8)
+    hipLaunchKernelGGL((skinny_gemm_kernel<KC, 8, MB>), grid, dim3(512), 0, stream, a);
+  else if (waves == 4)
+    hipLaunchKernelGGL((skinny_gemm_kernel<KC, 4, MB>), grid, dim3(256), 0, stream, a);
+  else if constexpr (MB == 4 && KC == 1024)
+    hipLaunchKernelGGL((skinny_gemm_kernel<KC, 6, MB>), grid, dim3(384), 0, stream, a);
+  return hipGetLastError();
+}
+
+template <int KC>
+hipError_t launch_gemm(const SkinnyGemmArgs &a, int waves, hipStream_t stream) {
+  if (a.M <= 16) return launch_gemm_tile<KC, 1>(a, waves, stream);
+  if (a.M <= 32) return launch_gemm_tile<KC, 2>(a, waves, stream);
+  if constexpr (KC <= 1024) return launch_gemm_tile<KC, 4>(a, waves, stream);
+  return hipErrorInvalidValue;  // 64 rows of x past 1024 columns do not fit the LDS (checked by the caller)
+}
+
 hipError_t launch_skinny_gemm(const SkinnyGemmArgs &a, int kc, hipStream_t stream) {
   const int cus = device_cu_count();
   const int splits = a.K / kc, mt = (a.M + 63) / 64;
   int waves;
-  if (kc == 1024) {
+  if (kc == 1024 && a.M > 32) {
     // One workgroup per CU (the x chunk takes 132 KB of LDS): the shape whose
     // busiest CU streams the fewest weight rows. (gate|up at C5, N 12288 on
     // 256 CUs: 6 waves, one 192 KB workgroup per CU, 14.7-15.1 us against
@@ -493,17 +562,13 @@ hipError_t launch_skinny_gemm(const SkinnyGemmArgs &a, int kc, hipStream_t strea
     const bool wide = a.N % 128 == 0 && 4 * (int64_t)(a.N / 128) * splits * mt >= 3 * (int64_t)cus;
     waves = wide ? 8 : 4;
   }
-  const dim3 grid((unsigned)(a.N / (16 * waves)), (unsigned)splits, (unsigned)mt);
-#define TT_GEMM_LAUNCH(KC, W) hipLaunchKernelGGL((skinny_gemm_kernel<KC, W>), grid, dim3(64 * W), 0, stream, a)
-  if (kc == 256) {
-    if (waves == 8) TT_GEMM_LAUNCH(256, 8); else TT_GEMM_LAUNCH(256, 4);
-  } else if (kc == 512) {
-    if (waves == 8) TT_GEMM_LAUNCH(512, 8); else TT_GEMM_LAUNCH(512, 4);
-  } else {
-    if (waves == 8) TT_GEMM_LAUNCH(1024, 8); else if (waves == 6) TT_GEMM_LAUNCH(1024, 6); else TT_GEMM_LAUNCH(1024, 4);
+  switch (kc) {
+    case 256: return launch_gemm<256>(a, waves, stream);
+    case 512: return launch_gemm<512>(a, waves, stream);
+    case 1024: return launch_gemm<1024>(a, waves, stream);
+    case 1280: return launch_gemm<1280>(a, waves, stream);
+    default: return hipErrorInvalidValue;
   }
-#undef TT_GEMM_LAUNCH
-  return hipGetLastError();
 }
 
 hipError_t launch_reduce_bf16(const float *P, int S, int64_t MN, uint16_t *y, hipStream_t stream) {
@@ -518,34 +583,39 @@ hipError_t launch_add_rmsnorm(float *x, const float *P, int S, int M, int C, con
 #define TT_ADD_RMSNORM_LAUNCH(n, smax)                                                                       \
   do {                                                                                                      \
     if (C % 1024 == 0)                                                                                      \
-      hipLaunchKernelGGL((add_rmsnorm_kernel<n, smax, false>), dim3(M), dim3(256), 0, stream, x, P, S, MN, w, eps, \
+      hipLaunchKernelGGL((add_rmsnorm_kernel<n, smax, false, 256>), dim3(M), dim3(256), 0, stream, x, P, S, MN, w, eps, \
                          y, C);                                                                             \
     else                                                                                                    \
-      hipLaunchKernelGGL((add_rmsnorm_kernel<n, smax, true>), dim3(M), dim3(256), 0, stream, x, P, S, MN, w, eps, \
+      hipLaunchKernelGGL((add_rmsnorm_kernel<n, smax, true, 256>), dim3(M), dim3(256), 0, stream, x, P, S, MN, w, eps, \
                          y, C);                                                                             \
   } while (0)
-#define TT_ADD_RMSNORM_CASE(n)                  \
-  case n:                                       \
-    if (S <= 4)                                 \
-      TT_ADD_RMSNORM_LAUNCH(n, 4);              \
-    else if (S <= 8 && n <= 4)                  \
-      TT_ADD_RMSNORM_LAUNCH(n, (n <= 4 ? 8 : 4)); \
-    else                                        \
-      TT_ADD_RMSNORM_LAUNCH(n, (n <= 2 ? 16 : 4)); \
-    break;
-  switch ((C + 1023) / 1024) {  // C a multiple of 4 in [4, 8192], checked by the caller
-    TT_ADD_RMSNORM_CASE(1)
-    TT_ADD_RMSNORM_CASE(2)
-    TT_ADD_RMSNORM_CASE(3)
-    TT_ADD_RMSNORM_CASE(4)
-    TT_ADD_RMSNORM_CASE(5)
-    TT_ADD_RMSNORM_CASE(6)
-    TT_ADD_RMSNORM_CASE(7)
-    TT_ADD_RMSNORM_CASE(8)
-    default:
-      return hipErrorInvalidValue;
+  // C a multiple of 4 in [4, 8192], checked by the caller
+  if (C > 2048 && S > 4) {
+    const bool whole = C % 4096 == 0;
+#define TT_ADD_RMSNORM_WIDE(n, smax, mask)                                                                          \
+  hipLaunchKernelGGL((add_rmsnorm_kernel<n, smax, mask, 1024>), dim3(M), dim3(1024), 0, stream, x, P, S, MN, w, eps, \
+                     y, C)
+    if (C <= 4096) {
+      if (whole) TT_ADD_RMSNORM_WIDE(1, 16, false); else TT_ADD_RMSNORM_WIDE(1, 16, true);
+    } else {
+      if (whole) TT_ADD_RMSNORM_WIDE(2, 8, false); else TT_ADD_RMSNORM_WIDE(2, 8, true);
+    }
+#undef TT_ADD_RMSNORM_WIDE
+  } else if (C <= 1024) {
+    if (S <= 4) TT_ADD_RMSNORM_LAUNCH(1, 4); else if (S <= 8) TT_ADD_RMSNORM_LAUNCH(1, 8); else TT_ADD_RMSNORM_LAUNCH(1, 16);
+  } else if (C <= 2048) {
+    if (S <= 4) TT_ADD_RMSNORM_LAUNCH(2, 4); else if (S <= 8) TT_ADD_RMSNORM_LAUNCH(2, 8); else TT_ADD_RMSNORM_LAUNCH(2, 16);
+  } else {
+    switch ((C + 1023) / 1024) {  // S <= 4
+      case 3: TT_ADD_RMSNORM_LAUNCH(3, 4); break;
+      case 4: TT_ADD_RMSNORM_LAUNCH(4, 4); break;
+      case 5: TT_ADD_RMSNORM_LAUNCH(5, 4); break;
+      case 6: TT_ADD_RMSNORM_LAUNCH(6, 4); break;
+      case 7: TT_ADD_RMSNORM_LAUNCH(7, 4); break;
+      case 8: TT_ADD_RMSNORM_LAUNCH(8, 4); break;
+      default: return hipErrorInvalidValue;
+    }
   }
-#undef TT_ADD_RMSNORM_CASE
 #undef TT_ADD_RMSNORM_LAUNCH
   return hipGetLastError();
 }
@@ -562,17 +632,24 @@ int swiglu_row_blocks(int64_t I) {
   return 2;
 }
 
+template <int K, int MB>
+hipError_t launch_swiglu_tile(const SwigluGemmArgs &a, hipStream_t stream) {
+  const int nb = swiglu_row_blocks(a.I);
+  const dim3 grid((unsigned)(a.I / (8 * nb)), 1, (unsigned)((a.M + 16 * MB - 1) / (16 * MB)));
+  if (nb == 3)
+    hipLaunchKernelGGL((swiglu_gemm_kernel<K, 3, MB>), grid, dim3(128 * 3), 0, stream, a);
+  else if (nb == 4)
+    hipLaunchKernelGGL((swiglu_gemm_kernel<K, 4, MB>), grid, dim3(128 * 4), 0, stream, a);
+  else
+    hipLaunchKernelGGL((swiglu_gemm_kernel<K, 2, MB>), grid, dim3(128 * 2), 0, stream, a);
+  return hipGetLastError();
+}
+
 template <int K>
 hipError_t launch_swiglu_k(const SwigluGemmArgs &a, hipStream_t stream) {
-  const int nb = swiglu_row_blocks(a.I);
-  const dim3 grid((unsigned)(a.I / (8 * nb)), 1, (unsigned)((a.M + 63) / 64));
-  if (nb == 3)
-    hipLaunchKernelGGL((swiglu_gemm_kernel<K, 3>), grid, dim3(128 * 3), 0, stream, a);
-  else if (nb == 4)
-    hipLaunchKernelGGL((swiglu_gemm_kernel<K, 4>), grid, dim3(128 * 4), 0, stream, a);
-  else
-    hipLaunchKernelGGL((swiglu_gemm_kernel<K, 2>), grid, dim3(128 * 2), 0, stream, a);
-  return hipGetLastError();
+  if (a.M <= 16) return launch_swiglu_tile<K, 1>(a, stream);
+  if (a.M <= 32) return launch_swiglu_tile<K, 2>(a, stream);
+  return launch_swiglu_tile<K, 4>(a, stream);
 }
 
 hipError_t launch_swiglu_gemm(const SwigluGemmArgs &a, hipStream_t stream) {

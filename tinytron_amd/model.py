@@ -294,16 +294,32 @@ class GPT(nn.Module):
     def _k_chunk(k: int) -> int:
         return 512 if k % 512 == 0 else (256 if k % 256 == 0 else 0)
 
-    @staticmethod
-    def _k_chunk_wide(k: int) -> int:
-        """Split for the gate|up GEMM: its N fills every CU at 1024-wide chunks,
-        which halve the partials that SwiGLU reads."""
-        return 1024 if k % 1024 == 0 else GPT._k_chunk(k)
+    def _chunks(self, B: int) -> tuple:
+        """Split-K chunk widths of a B-row decode step's projections (q|k|v,
+        c_proj, gate|up, down). 512 where it divides K, except:
 
-    @staticmethod
-    def _k_chunk_small(k: int) -> int:
-        """Split for the square c_proj GEMM: more, shorter splits keep every CU streaming."""
-        return 256 if k % 256 == 0 else 0
+        * q|k|v of up to 32 rows with more than FUSED_STEP_MAX_SPLITS such
+          splits: 1280-wide chunks if those are few enough for the fused
+          attention step (K 5120, 5 rows: 14.8 us against 15.9, and no RoPE +
+          append launch);
+        * c_proj whose 512-wide chunks would not cover 3/4 of the CUs: 256 (K
+          2048, 64 rows: 4.6 us against 5.3; at K 5120, 400 workgroups, 512 is
+          the faster one: 15.4 us against 19.6);
+        * gate|up: 1024, with half the partials, for up to 16 rows (equal
+          time: K 5120, N 27648, 5 rows 54.7 us against 54.4) and for wider
+          batches where one workgroup per CU takes it whole (N 12288, K 2048:
+          14.7 us against 16.1; N 27648, K 5120, 64 rows: 89 us against 72)."""
+        c = self.config
+        C, inter, cus = c.hidden_size, c.intermediate_size, 256
+        qkv = self._k_chunk(C)
+        if B <= 32 and C // qkv > ops.FUSED_STEP_MAX_SPLITS and C % 1280 == 0 \
+                and C // 1280 <= ops.FUSED_STEP_MAX_SPLITS:
+            qkv = 1280
+        o = 256 if C % 512 or 4 * (C // 128) * (C // 512) < 3 * cus else 512
+        gu = self._k_chunk(C)
+        if C % 1024 == 0 and (B <= 16 or (B > 32 and (2 * inter // 96) * (C // 1024) <= cus)):
+            gu = 1024
+        return qkv, o, gu, self._k_chunk(inter)
 
     def _fused_decode_ok(self, cache, B: int) -> bool:
         c = self.config
@@ -313,7 +329,7 @@ class GPT(nn.Module):
         n_qkv = (c.num_attention_heads + 2 * c.num_key_value_heads) * D
         return (c.hidden_size <= 8192 and n_qkv % 64 == 0
                 and (2 * c.intermediate_size) % 64 == 0 and self._k_chunk(c.hidden_size) > 0
-                and self._k_chunk_small(c.hidden_size) > 0 and self._k_chunk(c.intermediate_size) > 0
+                and self._k_chunk(c.intermediate_size) > 0
                 and all(_is_fused_cache(cache.get_layer_cache(i)) for i in range(len(self.blocks))))
 
     def _stacked_weights(self, i: int):
@@ -359,10 +375,9 @@ class GPT(nn.Module):
         c = self.config
         D = c.hidden_size // c.num_attention_heads
         n_qkv = (c.num_attention_heads + 2 * c.num_key_value_heads) * D
-        sizes = [(c.hidden_size // self._k_chunk(c.hidden_size)) * n_qkv,
-                 (c.hidden_size // self._k_chunk_wide(c.hidden_size)) * 2 * c.intermediate_size,
-                 (c.hidden_size // self._k_chunk_small(c.hidden_size)) * c.hidden_size,
-                 (c.intermediate_size // self._k_chunk(c.intermediate_size)) * c.hidden_size]
+        qkv, o, gu, down = self._chunks(B)
+        sizes = [(c.hidden_size // qkv) * n_qkv, (c.hidden_size // gu) * 2 * c.intermediate_size,
+                 (c.hidden_size // o) * c.hidden_size, (c.intermediate_size // down) * c.hidden_size]
         need = B * max(sizes)
         key = (str(device), B)
         buf = self._decode_bufs.get(key)
@@ -379,8 +394,7 @@ class GPT(nn.Module):
         C, Hq, Hkv = c.hidden_size, c.num_attention_heads, c.num_key_value_heads
         D = C // Hq
         eps = self.lnf.variance_epsilon
-        kc_c, kc_i, kc_o = self._k_chunk(C), self._k_chunk(c.intermediate_size), self._k_chunk_small(C)
-        kc_gu = self._k_chunk_wide(C)
+        kc_c, kc_o, kc_gu, kc_i = self._chunks(B)
         swiglu_fused = self._swiglu_fused()
         first = cache.get_layer_cache(0)
         lens = first.seq_lens_host
@@ -492,7 +506,9 @@ class GPT(nn.Module):
         x, h, y, a = bufs
         n = len(layers)
         arr = (_lib.DecodeLayer * n)()
-        kc_gu = 0 if self._swiglu_fused() else self._k_chunk_wide(C)
+        kc_qkv, kc_o, kc_gu, kc_down = self._chunks(B)
+        if self._swiglu_fused():
+            kc_gu = 0
         for i, (layer, st, w) in enumerate(zip(layers, steps, weights)):
             lay = layer.layout
             nxt = self.blocks[i + 1].ln_1.weight if i + 1 < n else self.lnf.weight
@@ -506,7 +522,7 @@ class GPT(nn.Module):
             L.ln2_weight, L.next_norm_weight = self.blocks[i].ln_2.weight.data_ptr(), nxt.data_ptr()
             L.eps = self.lnf.variance_epsilon
             L.batch, L.hidden, L.intermediate, L.num_q_heads, L.num_kv_heads, L.head_dim = B, C, I, Hq, Hkv, D
-            L.kc_qkv, L.kc_o, L.kc_gu, L.kc_down = self._k_chunk(C), self._k_chunk_small(C), kc_gu, self._k_chunk(I)
+            L.kc_qkv, L.kc_o, L.kc_gu, L.kc_down = kc_qkv, kc_o, kc_gu, kc_down
             L.fp8_cache = 1 if lay.kind == "fp8" else 0
             L.rope_table, L.rope_table_len = table.data_ptr(), table.shape[0]
             L.positions, L.lens_out = st[0].data_ptr(), st[1].data_ptr()
