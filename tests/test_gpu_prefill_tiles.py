@@ -7,7 +7,7 @@ attention tests (2e-3 + 2e-2 |ref|).
 """
 import pytest
 
-pytest.importorskip("torch")
+torch = pytest.importorskip("torch")
 
 from tests.test_gpu_prefill_attention import check, run_prefill
 
@@ -28,3 +28,43 @@ pytestmark = pytest.mark.gpu
 ])
 def test_prefill_workgroup_edges(past, new, Hq, Hkv, D, kw):
     check(*run_prefill(past, new, Hq=Hq, Hkv=Hkv, D=D, seed=D + len(past), **kw))
+
+
+@pytest.mark.parametrize("G,D,fp8", [(4, 64, False), (1, 64, False), (16, 128, False), (3, 32, False),
+                                     (4, 64, True), (8, 128, True)])
+@pytest.mark.parametrize("past,token", [(0, 40), (0, 79), (21, 33), (50, 14)])
+def test_infinite_value_of_a_later_token_stays_there(G, D, fp8, past, token):
+    # Value row `token` of a chunk of 80 is infinite (fp8: its codes NaN, its scale infinite). The tokens
+    # of earlier waves (32 // G tokens each) share its 64-key tile and must not see it, bit for bit.
+    from tinytron_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(D + G)
+    Hkv, new, cap = 2, 80, 144
+    rows = Hkv * cap
+    q = torch.randn(1, Hkv * G, new, D, generator=g, device="cuda").bfloat16()
+    kw = {}
+    if fp8:
+        k, v = (torch.randn(rows, D, generator=g, device="cuda").to(torch.float8_e4m3fn).view(torch.uint8) for _ in "kv")
+        scale = torch.rand(2 * rows, generator=g, device="cuda") + 0.5  # groups of 16 K scales, then 16 V scales
+        kw = dict(k_scale=scale, v_scale=scale[16:])
+    else:
+        k, v = (torch.randn(rows, D, generator=g, device="cuda").bfloat16() for _ in "kv")
+
+    def run():
+        kv = ops.KVLayout(k=k.view(-1), v=v.view(-1), strides=(Hkv * cap * D, 16 * D, cap * D), num_heads=Hkv,
+                          head_dim=D, page_size=16, capacity=cap, kind="fp8" if fp8 else "bf16", **kw)
+        return ops.prefill_attention(q, kv, torch.tensor([past], dtype=torch.int32, device="cuda"), past + new)
+
+    plain = run()
+    for h in range(Hkv):
+        r = h * cap + past + token
+        if fp8:
+            v[r] = 0x7F
+            scale[r + r // 16 * 16 + 16] = float("inf")
+        else:
+            v[r] = float("inf")
+    got = run()
+    first = token // (32 // G) * (32 // G)  # of the token's wave
+    assert torch.isfinite(plain.float()).all()
+    assert torch.equal(got[:, :first], plain[:, :first])
+    assert not torch.isfinite(got[:, token:].float()).any()

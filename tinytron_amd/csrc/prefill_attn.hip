@@ -26,6 +26,12 @@
 //                 of the 16 contracted keys is the one S^T's layout leaves in
 //                 each lane's registers, used for V as well: P needs no shuffle.
 //
+// Tiles below the workgroup's first token are whole for every column and run
+// in a loop without masks; the others run in a loop of their own, in which a
+// wave leaves out the 32 keys of Q K^T and the 16-key steps of P V past its last
+// token and takes V past it as zero: the tile holds values of later waves'
+// tokens, and an infinity or NaN there would reach this wave's columns as 0 x inf.
+//
 // Bound: the shared issue of VALU and matrix instructions. Per 32 x 32 block at
 // D 64 a wave issues ~125 VALU instructions (16 exponentials; the P split is 48,
 // the sums and the maxima 24) and 12 MFMAs; measured, 8 MFMAs and 64 FMAs of one
@@ -43,6 +49,7 @@
 // With many pairs, all query blocks of one (sequence, KV head) run on one XCD,
 // whose L2 keeps the pair's K/V for them (prefill_group).
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_tiles.h"
 #include "tt_internal.h"
@@ -216,24 +223,24 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
   const int t_first = grp * wg_tokens + wave * a.qt;
   const int t_end = min(t_first + a.qt, nb);
   const int Lw = t_first < nb ? __builtin_amdgcn_readfirstlane(min(pos0 + t_end, L)) : 0;
-  // smallest key limit of the wave's valid columns (its first token's): key
-  // ranges below it are whole for every column and skip the mask
-  const int lim_min = __builtin_amdgcn_readfirstlane(min(pos0 + t_first + 1, L));
+  // keys below the workgroup's first token's limit are whole for every column
+  const int lim_min = __builtin_amdgcn_readfirstlane(min(pos0 + grp * wg_tokens + 1, L));
 
   const int G = a.group;
   const int tq = n / G;
   const int head = n - tq * G;
   const int tok = t_first + tq;
   const bool col_valid = tq < a.qt && tok < t_end;
-  const int lim = col_valid ? min(pos0 + tok + 1, L) : 1;  // keys this column may see
   bf16x8 qf[D / 16];
   const uint16_t *q = static_cast<const uint16_t *>(a.q) + (int64_t)b * a.q_sb + (int64_t)(hk * G + head) * a.q_sh +
                       (int64_t)tok * a.q_st;
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) {
     const int d = 16 * s + 8 * half;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (col_valid && (!kPad || d < hd)) v = *reinterpret_cast<const u32x4 *>(q + d);
+    // loaded without a branch: from the tensor's first row where there is no value
+    const bool in = col_valid && (!kPad || d < hd);
+    u32x4 v = *reinterpret_cast<const u32x4 *>(in ? q + d : static_cast<const uint16_t *>(a.q));
+    if (!in) v = u32x4{0u, 0u, 0u, 0u};
     qf[s] = __builtin_bit_cast(bf16x8, v);
   }
   f32x16 o[D / 32];
@@ -265,7 +272,16 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
   const int vj = (lane >> 2) & 3, vq = lane & 3;  // key 4 half + vj, columns 4 vq .. + 3 of a 16-column group
   const int va0 = (4 * half + vj) * SH::kRowBytes +
                   16 * (v_swizzle<D>(4 * half + vj) + 2 * ((lane >> 4) & 1) + (vq >> 1)) + 8 * (vq & 1);
-  for (int i = 0; i < tiles; ++i) {
+  // Between tiles one register holds both offsets (ka0 < 2^13, va0 < 2^12) and
+  // the column's token in the wave (and the lane's half): with more, 128 registers do not do (a
+  // reload in the loop would wait for the next tile's loads).
+  const uint32_t packed = ka0 | (uint32_t)va0 << 13 | (uint32_t)(col_valid ? tq : 0) << 25 |
+                          (uint32_t)half << 31;
+  // One tile. A tile that some column may see only in part (kEdge) has code of its own:
+  // branches between the P V steps keep one step's softmax from running beside another's
+  // MFMAs (in every tile they cost 1-17 % of the kernel).
+  auto step = [&](int i, auto edge_tile) {
+    constexpr bool kEdge = decltype(edge_tile)::value;
     const bool more = i + 1 < tiles;
     if (more) {
       if ((kKeys * (i + 1)) % 1024 == 0) fetch_entries(i + 1);
@@ -277,34 +293,45 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
     const float *sc = reinterpret_cast<const float *>(lds + SH::kScaleAt) + (i & 1) * kKeys;
     const int t0 = kKeys * i;
     if (t0 < Lw) {  // uniform
+      uint32_t pk = packed;
+      asm volatile("" : "+v"(pk));
+      const int ka = pk & 0x1fff, va = (pk >> 13) & 0xfff;
+      const int quad = 4 * (int)(pk >> 31);
       f32x16 S[NU];
 #pragma unroll
       for (int u = 0; u < NU; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) S[u][r] = 0.f;
+      if (!kEdge || Lw - t0 > 32) {  // uniform
 #pragma unroll
-      for (int s = 0; s < D / 16; ++s)
+        for (int s = 0; s < D / 16; ++s)
 #pragma unroll
-        for (int u = 0; u < NU; ++u) {  // two independent chains
-          const bf16x8 kf = *reinterpret_cast<const bf16x8 *>(kb + 32 * u * SH::kRowBytes + (ka0 ^ (32 * s)));
-          S[u] = mfma32(kf, qf[s], S[u]);
-        }
+          for (int u = 0; u < NU; ++u) {  // two independent chains
+            const bf16x8 kf = *reinterpret_cast<const bf16x8 *>(kb + 32 * u * SH::kRowBytes + (ka ^ (32 * s)));
+            S[u] = mfma32(kf, qf[s], S[u]);
+          }
+      } else {  // no token of the wave sees the second half
+#pragma unroll
+        for (int s = 0; s < D / 16; ++s)
+          S[0] = mfma32(*reinterpret_cast<const bf16x8 *>(kb + (ka ^ (32 * s))), qf[s], S[0]);
+      }
       if constexpr (kFP8) {  // K scales (times the softmax scale: log2 units)
 #pragma unroll
         for (int u = 0; u < NU; ++u)
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
-            const f32x4 kc = *reinterpret_cast<const f32x4 *>(sc + 32 * u + 8 * x + 4 * half);
+            const f32x4 kc = *reinterpret_cast<const f32x4 *>(sc + 32 * u + 8 * x + quad);
 #pragma unroll
             for (int r = 0; r < 4; ++r) S[u][4 * x + r] *= kc[r];
           }
       }
-      if (t0 + kKeys > lim_min) {  // uniform: a tile that some column sees only in part
+      if constexpr (kEdge) {
+        const int lim = min(pos0 + t_first + (int)((pk >> 25) & 31) + 1, L);  // keys this column may see
 #pragma unroll
         for (int u = 0; u < NU; ++u)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int key = t0 + 32 * u + 8 * (r >> 2) + (r & 3) + 4 * half;
+            const int key = t0 + 32 * u + 8 * (r >> 2) + (r & 3) + quad;
             S[u][r] = key < lim ? S[u][r] : kNegInf;
           }
       }
@@ -330,6 +357,7 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
       for (int u = 0; u < NU; ++u)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
+          if (kEdge && t0 + 32 * u + 16 * t >= Lw) continue;  // uniform: keys past the wave's last token
           bf16x8 vf[D / 32];
 #pragma unroll
           for (int c = 0; c < D / 32; ++c) {
@@ -337,9 +365,21 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
 #pragma unroll
             for (int w = 0; w < 2; ++w)
               part[w] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4t *)(
-                  vb + (32 * u + 16 * t + 8 * w) * SH::kRowBytes + (va0 ^ (64 * c))));
+                  vb + (32 * u + 16 * t + 8 * w) * SH::kRowBytes + (va ^ (64 * c))));
             vf[c] = bf16x8{part[0][0], part[0][1], part[0][2], part[0][3],
                            part[1][0], part[1][1], part[1][2], part[1][3]};
+          }
+          if (kEdge && t0 + 32 * u + 16 * t + 16 > Lw) {  // uniform: V past the wave's last token is zero
+            const int left = Lw - (t0 + 32 * u + 16 * t + quad);
+            u32x4 keep;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const int r = 8 * (w >> 1) + 2 * (w & 1);
+              keep[w] = (r < left ? 0xffffu : 0u) | (r + 1 < left ? 0xffff0000u : 0u);
+            }
+#pragma unroll
+            for (int c = 0; c < D / 32; ++c)
+              vf[c] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, vf[c]) & keep);
           }
           float p[8];
 #pragma unroll
@@ -350,9 +390,12 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
           if constexpr (kFP8) {  // fold the V scales in; a row past the end has scale and P zero
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
-              const f32x4 vc = *reinterpret_cast<const f32x4 *>(sc + 2 * kKeys + 32 * u + 16 * t + 8 * x + 4 * half);
+              const f32x4 vc = *reinterpret_cast<const f32x4 *>(sc + 2 * kKeys + 32 * u + 16 * t + 8 * x + quad);
 #pragma unroll
-              for (int r = 0; r < 4; ++r) p[4 * x + r] *= vc[r];
+              for (int r = 0; r < 4; ++r) {
+                const float pv = p[4 * x + r] * vc[r];
+                p[4 * x + r] = kEdge && p[4 * x + r] == 0.f ? 0.f : pv;  // a masked token's scale may be infinite
+              }
             }
           }
           bf16x8 hi, lo;
@@ -367,19 +410,27 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
     // the other buffer's readers are done since the last barrier
     if (more) stage_store<D, kFP8>(a, st, lds, (i + 1) & 1);
     __syncthreads();
-  }
+  };
+  int i = 0;
+  for (const int whole = min(lim_min / kKeys, tiles); i < whole; ++i) step(i, std::false_type{});
+  for (; i < tiles; ++i) step(i, std::true_type{});
 
   // normalise and write: the lane's column, head_dim entries 32 c + 8 i + 4 half .. + 3
   const float sum = l + __shfl_xor(l, 32, 64);
   const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-  if (!col_valid) return;
-  uint16_t *out = static_cast<uint16_t *>(a.out) + (int64_t)b * a.o_sb + (int64_t)tok * a.o_st +
-                  (int64_t)(hk * G + head) * a.o_sh;
+  // the column again from the lane: its token and head would take registers through the loop
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int tq_out = (ln & 31) / G;
+  const int tok_out = t_first + tq_out;
+  if (tq_out >= a.qt || tok_out >= t_end) return;
+  uint16_t *out = static_cast<uint16_t *>(a.out) + (int64_t)b * a.o_sb + (int64_t)tok_out * a.o_st +
+                  (int64_t)(hk * G + (ln & 31) - tq_out * G) * a.o_sh;
 #pragma unroll
   for (int c = 0; c < D / 32; ++c)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int d0 = 32 * c + 8 * i + 4 * half;
+      const int d0 = 32 * c + 8 * i + 4 * (ln >> 5);
       if (kPad && d0 >= hd) continue;  // columns past head_dim (hd is a multiple of 8)
       const uint2 w = make_uint2(pack_bf16x2(o[c][4 * i] * inv, o[c][4 * i + 1] * inv),
                                  pack_bf16x2(o[c][4 * i + 2] * inv, o[c][4 * i + 3] * inv));
