@@ -30,6 +30,15 @@
 //          distribution as torch.multinomial over softmax(filtered), not the
 //          same random stream.
 //
+// Bound: the whole-row path by instruction issue on the row's one CU (32 values a
+// thread at V 32000, each pass several instructions a value) and the barriers of
+// the four digit passes. So y is divided once and kept, the sum of all masses comes
+// from the first digit's histogram, log Z and the draw's sums from one pass, and
+// the draw finds its place by a prefix sum over a wave's lanes. With a division in each of
+// nine passes before -> now (us a call): [64, 32000] bf16, top-p 0.9, temperature
+// 0.8 103.1 -> 56.3; fp32 92.4 -> 50.5; [5, 4096] 34.2 -> 24.4; [128, 50304]
+// (64 values a thread: raw pairs stay, their y does not fit) 185.4 -> 121.4.
+//
 // Candidate path (2 <= top_k <= kCandSlots, no full log-probability rows,
 // V > kCandChunk): one workgroup per row leaves most CUs idle, so the row is
 // first cut into kCandChunk-logit chunks, each reduced on a workgroup of its
@@ -108,17 +117,6 @@ __device__ __forceinline__ u64 wave_sum_u64(u64 v) {
   return v;
 }
 
-__device__ __forceinline__ u64 block_sum_u64(u64 v, SampleShared &sh) {
-  v = wave_sum_u64(v);
-  if ((threadIdx.x & 63) == 0) sh.red[threadIdx.x >> 6][0] = v;
-  __syncthreads();
-  u64 t = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) t += sh.red[w][0];
-  __syncthreads();
-  return t;
-}
-
 // Sum in a fixed order: thread-sequential, xor butterfly, waves ascending.
 __device__ __forceinline__ float block_sum_f32(float v, SampleShared &sh) {
 #pragma unroll
@@ -133,8 +131,10 @@ __device__ __forceinline__ float block_sum_f32(float v, SampleShared &sh) {
 }
 
 // Wave 0: the largest digit d with sum_{d' >= d} hist[d'] >= need (the caller
-// guarantees the total reaches need); bc[0] = d, bc[1] = sum over d' > d.
-__device__ __forceinline__ void pick_digit(SampleShared &sh, u64 need) {
+// guarantees the total reaches need); bc[0] = d, bc[1] = sum over d' > d,
+// bc[3] = need. On the first digit need is need_of(the sum of all weights).
+template <class NeedFn>
+__device__ __forceinline__ void pick_digit(SampleShared &sh, u64 need, bool first, NeedFn need_of) {
   const int lane = threadIdx.x & 63;
   u64 h[4];
   u64 s = 0;
@@ -150,6 +150,11 @@ __device__ __forceinline__ void pick_digit(SampleShared &sh, u64 need) {
     if (lane >= off) incl += o;
   }
   const u64 excl = incl - s;
+  if (first) need = need_of(__shfl(incl, 63, 64));
+  if (lane == 0) {
+    sh.bc[0] = sh.bc[1] = 0;  // where no digit reaches need (no weight at all)
+    sh.bc[3] = need;
+  }
   if (incl >= need && excl < need) {
     u64 c = excl;
 #pragma unroll
@@ -164,12 +169,14 @@ __device__ __forceinline__ void pick_digit(SampleShared &sh, u64 need) {
   }
 }
 
-// The row as this thread holds it: fp32 values, or (bf16 logits) the raw
-// bf16 pairs, two per register, converted and divided by the temperature at
-// each use (the division is exact-rounded, so every pass sees the same y).
+// The row as this thread holds it: y = x / temperature in fp32 where the
+// registers allow (up to 32 values a thread), so that the exact-rounded division
+// is done once and not in every pass; otherwise the raw bf16 pairs, two per
+// register, converted and divided at each use (every pass sees the same y).
 template <int EPT, bool kF32>
 struct Row {
-  static constexpr int kRegs = kF32 ? EPT : EPT / 2;
+  static constexpr bool kValues = kF32 || EPT <= 32;
+  static constexpr int kRegs = kValues ? EPT : EPT / 2;
   uint32_t w[kRegs];
   int t;  // thread index
   int V;
@@ -177,11 +184,8 @@ struct Row {
   float temperature;
   __device__ __forceinline__ int index(int g, int e) const { return 8 * (t + kThreads * g) + e; }
   __device__ __forceinline__ float val(int j) const {
-    float x;
-    if (kF32)
-      x = __uint_as_float(w[j]);
-    else
-      x = __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
+    if constexpr (kValues) return __uint_as_float(w[j]);
+    const float x = __uint_as_float((j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
     return apply_temp ? x / temperature : x;
   }
   // Start of a pass over the row: the values and the thread index count as
@@ -197,11 +201,13 @@ struct Row {
 
 // MSB-first radix select over the keys weighted by wfn(idx, y) (zero for
 // the -inf padding past V): the largest key kb with sum_{key >= kb} weight
-// >= need.
+// >= need, need = need_of(sum of all weights), from the first digit's histogram
+// (a pass over the row less than summing them first).
 // above = sum_{key > kb} weight, at = sum_{key == kb} weight.
-template <int EPT, bool kF32, class WeightFn>
-__device__ __forceinline__ uint32_t radix_select(SampleShared &sh, Row<EPT, kF32> &r, u64 need, WeightFn wfn,
-                                                 u64 &above, u64 &at) {
+template <int EPT, bool kF32, class NeedFn, class WeightFn>
+__device__ __forceinline__ uint32_t radix_select(SampleShared &sh, Row<EPT, kF32> &r, NeedFn need_of, WeightFn wfn,
+                                                 u64 &need, u64 &above, u64 &at) {
+  u64 left = 0;  // need less the weight above the prefix
   uint32_t prefix = 0, mask = 0;
   above = 0;
   at = 0;
@@ -231,13 +237,14 @@ __device__ __forceinline__ uint32_t radix_select(SampleShared &sh, Row<EPT, kF32
       sh.hist[threadIdx.x] = t;
     }
     __syncthreads();
-    if (threadIdx.x < 64) pick_digit(sh, need);
+    if (threadIdx.x < 64) pick_digit(sh, left, shift == 24, need_of);
     __syncthreads();
     const uint32_t d = (uint32_t)sh.bc[0];
     const u64 ab = sh.bc[1];
+    if (shift == 24) need = sh.bc[3];
+    left = sh.bc[3] - ab;
     at = sh.hist[d];
     above += ab;
-    need -= ab;
     prefix |= d << shift;
     mask |= 0xFFu << shift;
     __syncthreads();
@@ -245,41 +252,64 @@ __device__ __forceinline__ uint32_t radix_select(SampleShared &sh, Row<EPT, kF32
   return prefix;
 }
 
-// First index (in index order) at which the running sum of wfn(idx, y)
-// exceeds target (weights zero for the -inf padding); the caller guarantees
-// target < the total.
-template <int EPT, bool kF32, class WeightFn>
-__device__ __forceinline__ int find_first_exceeding(SampleShared &sh, Row<EPT, kF32> &r, u64 target, WeightFn wfn) {
-  constexpr int G = EPT / 8;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  u64 s[G];
-  r.pass();
+// The running sums that find_first_exceeding searches: s[g] = this thread's
+// weight in group g, sh.red[wave][g] = the wave's; returns the total.
+template <int G>
+__device__ __forceinline__ u64 share_sums(SampleShared &sh, const u64 (&s)[G]) {
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    s[g] = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      s[g] += wfn(r.index(g, e), r.val(8 * g + e));
-    }
     const u64 t = wave_sum_u64(s[g]);
-    if (lane == 0) sh.red[wave][g] = t;
+    if ((threadIdx.x & 63) == 0) sh.red[threadIdx.x >> 6][g] = t;
   }
   __syncthreads();
-  int gs = -1, ws = -1;
-  u64 cum = 0;
-#pragma unroll 1
-  for (int g = 0; g < G && gs < 0; ++g)
-#pragma unroll 1
-    for (int w = 0; w < kWaves; ++w) {
-      const u64 t = sh.red[w][g];
-      if (cum + t > target) {
-        gs = g;
-        ws = w;
-        break;
-      }
-      cum += t;
+  const int lane = threadIdx.x & 63;
+  u64 t = 0;
+#pragma unroll
+  for (int i = 0; i < (kWaves * G + 63) / 64; ++i)
+    if (64 * i + lane < kWaves * G) t += sh.red[(64 * i + lane) % kWaves][(64 * i + lane) / kWaves];
+  return wave_sum_u64(t);
+}
+
+// First index (in index order) at which the running sum of wfn(idx, y)
+// exceeds target (weights zero for the -inf padding), from share_sums; the
+// caller guarantees target < the total. Every wave finds the (group, wave) by a
+// prefix sum over its lanes: walked one by one, the up to 128 sums cost an LDS
+// round trip each.
+template <int EPT, bool kF32, class WeightFn>
+__device__ __forceinline__ int find_first_exceeding(SampleShared &sh, Row<EPT, kF32> &r, const u64 (&s)[EPT / 8],
+                                                    u64 target, WeightFn wfn) {
+  constexpr int G = EPT / 8;
+  constexpr int kPer = (kWaves * G + 63) / 64;  // (group, wave) sums per lane, in index order
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  u64 part[kPer], own = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int k = kPer * lane + i;
+    part[i] = k < kWaves * G ? sh.red[k % kWaves][k / kWaves] : 0;
+    own += part[i];
+  }
+  u64 run = own;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const u64 o = __shfl_up(run, off, 64);
+    if (lane >= off) run += o;
+  }
+  const u64 hit = __ballot(run > target);
+  if (threadIdx.x == 0) sh.bc[2] = 0;  // no hit: no weight at all
+  __syncthreads();
+  const int src = hit ? __builtin_ctzll(hit) : 0;
+  u64 cum = __shfl(run - own, src, 64);
+  int k = kPer * src;
+#pragma unroll
+  for (int i = 0; i + 1 < kPer; ++i) {
+    const u64 p = __shfl(part[i], src, 64);
+    if (k == kPer * src + i && cum + p <= target) {
+      cum += p;
+      ++k;
     }
+  }
+  const int gs = hit ? k / kWaves : -1, ws = hit ? k % kWaves : -1;
   if (wave == ws) {
     const u64 rel = target - cum;
     u64 sv = 0;
@@ -325,6 +355,8 @@ __device__ __forceinline__ int find_first_exceeding(SampleShared &sh, Row<EPT, k
 template <int EPT, bool kF32>
 __device__ __forceinline__ void load_row(const SampleArgs &a, int row, Row<EPT, kF32> &r) {
   constexpr int G = EPT / 8;
+  constexpr int kRaw = kF32 ? EPT : EPT / 2;
+  uint32_t w[kRaw];
   r.t = threadIdx.x;
   r.V = a.V;
   r.apply_temp = a.apply_temp;
@@ -347,15 +379,15 @@ __device__ __forceinline__ void load_row(const SampleArgs &a, int row, Row<EPT, 
 #pragma unroll
         for (int h = 0; h < kVec; ++h)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) r.w[(kF32 ? 8 : 4) * g + 4 * h + e] = raw[g][h][e];
+          for (int e = 0; e < 4; ++e) w[(kF32 ? 8 : 4) * g + 4 * h + e] = raw[g][h][e];
       } else {
 #pragma unroll
-        for (int j = 0; j < Row<EPT, kF32>::kRegs / G; ++j) r.w[(Row<EPT, kF32>::kRegs / G) * g + j] = kF32 ? 0xff800000u : 0xff80ff80u;
+        for (int j = 0; j < kRaw / G; ++j) w[(kRaw / G) * g + j] = kF32 ? 0xff800000u : 0xff80ff80u;
       }
     }
   } else {
 #pragma unroll
-    for (int j = 0; j < Row<EPT, kF32>::kRegs; ++j) r.w[j] = kF32 ? 0xff800000u : 0xff80ff80u;
+    for (int j = 0; j < kRaw; ++j) w[j] = kF32 ? 0xff800000u : 0xff80ff80u;
   }
   // The partial group (at most one per row), or every group for rows that
   // are not 16-byte aligned: element loads.
@@ -366,17 +398,27 @@ __device__ __forceinline__ void load_row(const SampleArgs &a, int row, Row<EPT, 
       if (kF32) {
         const float *src = reinterpret_cast<const float *>(rowp) + base;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) r.w[8 * g + e] = base + e < a.V ? __float_as_uint(src[e]) : 0xff800000u;
+        for (int e = 0; e < 8; ++e) w[8 * g + e] = base + e < a.V ? __float_as_uint(src[e]) : 0xff800000u;
       } else {
         const uint16_t *src = reinterpret_cast<const uint16_t *>(rowp) + base;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const uint32_t lo = base + 2 * e < a.V ? src[2 * e] : 0xff80u;
           const uint32_t hi = base + 2 * e + 1 < a.V ? src[2 * e + 1] : 0xff80u;
-          r.w[4 * g + e] = lo | (hi << 16);
+          w[4 * g + e] = lo | (hi << 16);
         }
       }
     }
+  }
+  if constexpr (Row<EPT, kF32>::kValues) {
+#pragma unroll
+    for (int j = 0; j < EPT; ++j) {
+      const float x = __uint_as_float(kF32 ? w[j] : (j & 1) ? (w[j >> 1] & 0xffff0000u) : (w[j >> 1] << 16));
+      r.w[j] = __float_as_uint(a.apply_temp ? x / a.temperature : x);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kRaw; ++j) r.w[j] = w[j];
   }
 }
 
@@ -795,9 +837,10 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
     if (greedy) {
       thrk = order_key(m);
     } else if (nfinite > a.top_k) {
-      u64 ab, at;
+      u64 need, ab, at;
       thrk = radix_select(
-          sh, r, (u64)a.top_k, [](int, float v) { return v > -INFINITY ? (u64)1 : (u64)0; }, ab, at);
+          sh, r, [&](u64) { return (u64)a.top_k; }, [](int, float v) { return v > -INFINITY ? (u64)1 : (u64)0; },
+          need, ab, at);
     }
   }
   auto kept_k = [&](float v) { return order_key(v) >= thrk; };
@@ -807,29 +850,28 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
   int ir = INT_MAX;
   const bool do_topp = a.apply_top_p && !fast;
   if (do_topp) {
-    u64 local = 0;
-    r.pass();
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = r.val(8 * g + e);
-        if (kept_k(v)) local += mass_of(v, m);
-      }
-    const u64 etot = block_sum_u64(local, sh);
-    const u64 T = (u64)((double)a.top_p * (double)etot);
-    u64 ab, at;
+    u64 need, ab, at;
     kb = radix_select(
-        sh, r, T + 1, [&](int, float v) { return kept_k(v) ? mass_of(v, m) : (u64)0; }, ab, at);
+        sh, r, [&](u64 etot) { return (u64)((double)a.top_p * (double)etot) + 1; },
+        [&](int, float v) { return kept_k(v) ? mass_of(v, m) : (u64)0; }, need, ab, at);
+    const u64 T = need - 1;
     const u64 eb = mass_of(key_value(kb), m);
     u64 keep_n = eb > 0 && T >= ab ? (T - ab) / eb : 0;
     if (ab == 0 && keep_n == 0) keep_n = 1;  // the first sorted token is always kept
     if (keep_n == 0) {
       ir = -1;
     } else if (eb > 0 && keep_n < at / eb) {
-      ir = find_first_exceeding(sh, r, keep_n - 1, [&](int, float v) {
-        return (kept_k(v) && order_key(v) == kb) ? (u64)1 : (u64)0;
-      });
+      auto tie = [&](int, float v) { return (kept_k(v) && order_key(v) == kb) ? (u64)1 : (u64)0; };
+      u64 s[G];
+      r.pass();
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        s[g] = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[g] += tie(r.index(g, e), r.val(8 * g + e));
+      }
+      share_sums<G>(sh, s);
+      ir = find_first_exceeding(sh, r, s, keep_n - 1, tie);
     }
   }
   auto keep = [&](int idx, float v) {
@@ -840,36 +882,32 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs a) {
     return k > kb || (k == kb && idx <= ir);
   };
 
-  // log Z over the kept tokens.
+  // log Z over the kept tokens, and their masses by group for the draw.
   float zl = 0.f;
+  u64 s[G];
   if (!fast) {
     r.pass();
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int g = 0; g < G; ++g) {
+      s[g] = 0;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int idx = r.index(g, e);
         const float v = r.val(8 * g + e);
-        if (keep(idx, v)) zl += expf(v - m);
+        if (keep(idx, v)) {
+          zl += expf(v - m);
+          s[g] += mass_of(v, m);
+        }
       }
+    }
   }
   const float logz = fast ? 0.f : logf(block_sum_f32(zl, sh));
 
   int tok = amax;
   if (!greedy) {
-    u64 local = 0;
-    r.pass();
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int idx = r.index(g, e);
-        const float v = r.val(8 * g + e);
-        if (keep(idx, v)) local += mass_of(v, m);
-      }
-    const u64 wtot = block_sum_u64(local, sh);
+    const u64 wtot = share_sums<G>(sh, s);
     const u64 target = __umul64hi(draw_u64(a.seed, a.offset, (u64)row), wtot);
-    tok = find_first_exceeding(sh, r, target, [&](int idx, float v) { return keep(idx, v) ? mass_of(v, m) : (u64)0; });
+    tok = find_first_exceeding(sh, r, s, target, [&](int idx, float v) { return keep(idx, v) ? mass_of(v, m) : (u64)0; });
   }
 
   // Outputs: the token (and its log-probability) from the thread holding it,
