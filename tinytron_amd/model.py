@@ -372,18 +372,16 @@ class GPT(nn.Module):
         return ent[1:]
 
     def _partials(self, device, B: int) -> torch.Tensor:
-        c = self.config
-        D = c.hidden_size // c.num_attention_heads
-        n_qkv = (c.num_attention_heads + 2 * c.num_key_value_heads) * D
-        qkv, o, gu, down = self._chunks(B)
-        sizes = [(c.hidden_size // qkv) * n_qkv, (c.hidden_size // gu) * 2 * c.intermediate_size,
-                 (c.hidden_size // o) * c.hidden_size, (c.intermediate_size // down) * c.hidden_size]
-        need = B * max(sizes)
         key = (str(device), B)
         buf = self._decode_bufs.get(key)
-        if buf is None or buf.numel() < need:
-            buf = torch.empty(need, dtype=torch.float32, device=device)
-            self._decode_bufs[key] = buf
+        if buf is None:
+            c = self.config
+            D = c.hidden_size // c.num_attention_heads
+            n_qkv = (c.num_attention_heads + 2 * c.num_key_value_heads) * D
+            qkv, o, gu, down = self._chunks(B)
+            sizes = [(c.hidden_size // qkv) * n_qkv, (c.hidden_size // gu) * 2 * c.intermediate_size,
+                     (c.hidden_size // o) * c.hidden_size, (c.intermediate_size // down) * c.hidden_size]
+            buf = self._decode_bufs[key] = torch.empty(B * max(sizes), dtype=torch.float32, device=device)
         return buf
 
     def _decode_step_fused(self, idx: torch.Tensor, cache, position_offset: int) -> torch.Tensor:
