@@ -2,7 +2,8 @@
 dispatch between the wide merge (at most 256 (sequence, KV head) segments) and
 the one-wave merge, and of the wide merge's own splits: one piece, fewer pieces
 than its four waves, one past a wave's 16-row batch, more than 64 pieces a wave
-(a lane each), sequences with nothing cached, every tile width and group size.
+(a lane each), sequences with nothing cached, every tile width and group size;
+NaN and infinite scores on both sides of the dispatch.
 
 Tolerance: the decode attention tests' (2e-3 + 2e-2 |ref|): the merge is the
 same fp32 sum of the same pieces in another order.
@@ -11,6 +12,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from tests.kv_inputs import sm_scale
 from tests.test_gpu_decode_attention import assert_close, run_case
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +35,32 @@ def test_merge_edges(lengths, Hq, Hkv, D, kw):
         assert (got[0] == 0).all()
         got, ref = got[1:], ref[1:]
     assert_close(got, ref)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("batch", [32, 33])  # 256 and 264 segments: the wide and the one-wave merge
+@pytest.mark.parametrize("lengths", [40, 700])
+def test_nan_and_infinite_scores_stay(D, batch, lengths):
+    # A NaN in q, a NaN in a cached key, an infinite score: NaN rows as softmax gives them, not zeros; a score
+    # of -inf drops its key. Every other row is as close as ever.
+    from tinytron_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(D + batch)
+    Hkv, G, cap = 8, 2, 704
+    q = torch.randn(batch, Hkv * G, D, generator=g, device="cuda").bfloat16()
+    k, v = (torch.randn(batch, Hkv, cap, D, generator=g, device="cuda").bfloat16() for _ in "kv")
+    q[1, 3, D - 1] = float("nan")
+    k[2, 4, lengths // 2, 0] = float("nan")
+    k[3, 5, lengths // 2, 1] = float("inf")  # +inf or -inf by the sign of each head's q[1]
+    q[3, 10, 1], q[3, 11, 1] = 1.0, -1.0
+    kv = ops.KVLayout(k=k.view(-1), v=v.view(-1), strides=(Hkv * cap * D, 16 * D, cap * D), num_heads=Hkv, head_dim=D,
+                      page_size=16, capacity=cap, kind="bf16")
+    lens = torch.full((batch,), lengths, dtype=torch.int32, device="cuda")
+    got = ops.decode_attention(q, kv, lens, lengths).float().cpu()
+    kc, vc = (x[:, :, :lengths].float().cpu().repeat_interleave(G, dim=1) for x in (k, v))
+    scores = (q.float().cpu()[:, :, None] * kc).sum(-1) * sm_scale(D)
+    ref = (torch.softmax(scores, -1)[..., None] * vc).sum(2)
+    nan = torch.isnan(ref)
+    assert nan[1, 3].all() and nan[2, 8:10].all() and nan[3, 10].all() and not nan[3, 11].any() and nan.sum() == 4 * D
+    assert torch.equal(torch.isnan(got), nan)
+    assert_close(got[~nan].numpy(), ref[~nan].numpy())

@@ -1303,7 +1303,9 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void decode_merge_wide_kernel(
       o += f * so[w][threadIdx.x];
       sum += f * sl[w];
     }
-    out[threadIdx.x] = f32_to_bf16_bits(sum > 0.f ? o / sum : 0.f);
+    // times an inverse, as the merge above: a NaN sum leaves o's NaN (a quotient selected by sum > 0 would hide it as 0)
+    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+    out[threadIdx.x] = f32_to_bf16_bits(o * inv);
   }
 }
 
