@@ -79,3 +79,31 @@ def test_infinite_value_of_a_later_token_stays_there():
     got, ref, _ = _run([0], [40], 4, 1, 64, False, seed=3, edit=edit)
     _check(got[:, :20], [r[:20] for r in ref], [20])
     assert np.all(np.isinf(got[0, 20:]))
+
+
+def _layer(B, Hkv, D, cap, seed):
+    from tinytron_amd.cache import LayerPagedKVCache
+
+    c = LayerPagedKVCache(B, Hkv, D, cap, 16, "cuda", torch.float32)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    c.layout.k.normal_(generator=g)
+    c.layout.v.normal_(generator=g)
+    return c, g
+
+
+def test_chunk_after_set_lengths_and_over_two_appends():
+    # The chunk ends at each sequence's length as the cache knows it, however the tokens came there.
+    from tinytron_amd import ops
+
+    B, Hq, Hkv, D, T = 2, 4, 2, 64, 6
+    c, g = _layer(B, Hkv, D, 64, 5)
+    q = torch.randn(B, Hq, T, D, generator=g, device="cuda")
+    c.set_lengths([40, 23])
+    got = c.prefill_attend(q, [6, 4])
+    assert torch.allclose(got, c.prefill_attend(q, [6, 4], kernel=False), rtol=1e-4, atol=1e-5)
+    table = ops.build_rope_table(64, D, dtype=torch.float32, device="cuda")
+    k = torch.randn(B, Hkv, 3, D, generator=g, device="cuda")
+    rot = torch.cat([c.rope_append(q[:, :, i:i + 3], k, k, table) for i in (0, 3)], dim=2)
+    assert c.seq_lens_host == [46, 29]
+    got = c.prefill_attend(rot, [6, 6])
+    assert torch.allclose(got, c.prefill_attend(rot, [6, 6], kernel=False), rtol=1e-4, atol=1e-5)

@@ -269,11 +269,13 @@ class _LayerCacheBase:
             nl = torch.tensor([int(n) for n in new_lens], dtype=torch.int32).to(prev.device, non_blocking=True)
             return ops.prefill_attention(q_rot, lay, prev, self.current_length, new_lens=nl, out=out)
         adds = [min(int(n), T) for n in new_lens]
-        if kernel and q_rot.dtype == torch.float32 and ops.prefill_f32_supported(lay, q_rot.shape[1]):
-            prev = self._lens_dev[1 - self._cur]
-            nl = torch.tensor(adds, dtype=torch.int32).to(prev.device, non_blocking=True)
-            return ops.prefill_attention_f32(q_rot, lay, prev, self.current_length, new_lens=nl, out=out)
         cached = [x - a for x, a in zip(self._host_lens, adds)]
+        if kernel and q_rot.dtype == torch.float32 and ops.prefill_f32_supported(lay, q_rot.shape[1]) \
+                and min(cached, default=0) >= 0:
+            # from the host's lengths, as row attention: the other length buffer holds those before the last
+            # append only (not after set_lengths, nor for a chunk that two appends wrote)
+            pos, nl = torch.tensor([cached, adds], dtype=torch.int32).to(q_rot.device, non_blocking=True)
+            return ops.prefill_attention_f32(q_rot, lay, pos, self.current_length, new_lens=nl, out=out)
         if self.workspace is None:
             self.workspace = ops.Workspace(q_rot.device)
         return ops.prefill_attention_rows(q_rot, lay, cached, adds, out=out, workspace=self.workspace)
