@@ -1303,9 +1303,8 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void decode_merge_wide_kernel(
       o += f * so[w][threadIdx.x];
       sum += f * sl[w];
     }
-    // times an inverse, as the merge above: a NaN sum leaves o's NaN (a quotient selected by sum > 0 would hide it as 0)
-    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-    out[threadIdx.x] = f32_to_bf16_bits(o * inv);
+    // zero only for an empty sum: a NaN sum (a NaN operand, an infinite score) stays NaN
+    out[threadIdx.x] = f32_to_bf16_bits(sum == 0.f ? 0.f : o / sum);
   }
 }
 
