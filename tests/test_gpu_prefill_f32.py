@@ -107,3 +107,46 @@ def test_chunk_after_set_lengths_and_over_two_appends():
     assert c.seq_lens_host == [46, 29]
     got = c.prefill_attend(rot, [6, 6])
     assert torch.allclose(got, c.prefill_attend(rot, [6, 6], kernel=False), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("form", ["q_strided", "q_token_major", "out_strided", "out_rows", "out_bf16"])
+def test_forms_that_row_attention_took(form):
+    # views of q and out that the kernel reads or writes directly, and those that go on taking row attention
+    B, Hq, Hkv, D, T = 2, 4, 2, 32, 7
+    c, g = _layer(B, Hkv, D, 48, 6)
+    c.set_lengths([40, 23])
+    q = torch.randn(B, Hq, T, D, generator=g, device="cuda")
+    ref = c.prefill_attend(q, [7, 4], kernel=False)
+    out = None
+    if form == "q_strided":
+        q = torch.stack([q, q + 1], -1)[..., 0]
+    elif form == "q_token_major":
+        q = q.transpose(1, 2).contiguous().transpose(1, 2)
+    elif form == "out_strided":
+        out = torch.empty(B, T, Hq, D, 2, device="cuda")[..., 1]
+    elif form == "out_rows":
+        out = torch.empty(B * T, Hq * D, device="cuda")
+    else:
+        out = torch.empty(B, T, D, Hq, device="cuda", dtype=torch.bfloat16).transpose(2, 3)
+    got = c.prefill_attend(q, [7, 4], out=out)
+    assert out is None or got is out
+    tol = dict(rtol=2.0 ** -8, atol=1e-5) if form == "out_bf16" else dict(rtol=1e-4, atol=1e-5)
+    assert torch.allclose(got.float().reshape(ref.shape), ref, **tol)
+
+
+def test_out_that_does_not_fit_is_refused():
+    from tinytron_amd import ops
+
+    c, g = _layer(2, 2, 32, 48, 7)
+    c.set_lengths([40, 23])
+    q = torch.randn(2, 4, 7, 32, generator=g, device="cuda")
+    pos = torch.tensor([33, 16], dtype=torch.int32, device="cuda")
+    for shape, dtype in [((2, 6, 4, 32), torch.float32), ((2, 7, 4, 32), torch.bfloat16), ((2, 7, 4, 36), torch.float32)]:
+        out = torch.empty(shape, dtype=dtype, device="cuda")
+        with pytest.raises(ValueError, match="out"):
+            ops.prefill_attention_f32(q, c.layout, pos, 40, out=out)
+    with pytest.raises(RuntimeError):
+        c.prefill_attend(q, [7, 7], out=torch.empty(2, 6, 4, 32, device="cuda"))
+    for where in (dict(out=torch.empty(2, 7, 4, 32)), dict(new_lens=torch.tensor([7, 7], dtype=torch.int32))):
+        with pytest.raises(ValueError):
+            ops.prefill_attention_f32(q, c.layout, pos, 40, **where)

@@ -529,7 +529,10 @@ int prefill_common(tt::CacheKind kind, const void *q, const int64_t q_strides[3]
     rc = check_contiguous_room(max_seq_len, head_dim, cache_strides, batch, num_kv_heads);
     if (rc != TT_OK) return rc;
   }
-  if (!f32) {
+  if (f32) {
+    TT_CHECK(aligned(q, 4) && aligned(k_cache, 4) && aligned(v_cache, 4) && aligned(out, 4), TT_ERR_INVALID_ARGUMENT,
+             "q, cache and out pointers must be aligned to their element size");
+  } else {
     TT_CHECK(aligned(q, 16) && aligned(k_cache, 16) && aligned(v_cache, 16), TT_ERR_INVALID_ARGUMENT,
              "q and cache pointers must be 16-byte aligned");
     TT_CHECK(q_strides[0] % 8 == 0 && q_strides[1] % 8 == 0 && q_strides[2] % 8 == 0, TT_ERR_INVALID_ARGUMENT,

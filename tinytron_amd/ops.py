@@ -779,6 +779,18 @@ def prefill_f32_supported(layout: KVLayout, num_q_heads: int) -> bool:
             and (layout.page_table is not None or layout.strides[1] == layout.page_size * layout.head_dim))
 
 
+def prefill_f32_takes(q: torch.Tensor, out: torch.Tensor | None, num_seqs: int) -> bool:
+    """Whether prefill_attention_f32 reads this q [num_seqs, H_q, T, D] and
+    writes this out as they are: head_dim contiguous, out fp32
+    [num_seqs, T, H_q, D] on q's device. prefill_attention_rows, which copies
+    where it must, takes every other form."""
+    if q.dim() != 4 or q.stride(-1) != 1 or q.shape[0] != num_seqs:
+        return False
+    B, Hq, T, D = q.shape
+    return out is None or (out.dtype == q.dtype and out.shape == (B, T, Hq, D) and out.stride(-1) == 1
+                           and out.device == q.device)
+
+
 def prefill_attention_f32(q: torch.Tensor, layout: KVLayout, positions: torch.Tensor, max_seq_len: int,
                           new_lens: torch.Tensor | None = None, out: torch.Tensor | None = None,
                           sm_scale: float | None = None) -> torch.Tensor:
@@ -786,11 +798,14 @@ def prefill_attention_f32(q: torch.Tensor, layout: KVLayout, positions: torch.Te
     without autocast, attn.py:321-341); rows t >= new_lens[b] are zeros."""
     if q.dtype != torch.float32 or layout.kind != "f32":
         raise ValueError("prefill_attention_f32 takes fp32 q with an fp32 cache")
+    if not prefill_f32_takes(q, out, q.shape[0]):
+        raise ValueError("prefill_attention_f32 takes q [B, H_q, T, D] and an fp32 out [B, T, H_q, D] on its device, "
+                         "both contiguous in head_dim")
     return _prefill_attention(q, layout, positions, max_seq_len, new_lens, out, sm_scale)
 
 
 def _prefill_attention(q, layout, positions, max_seq_len, new_lens, out, sm_scale):
-    _require_cuda(q, layout.k, layout.v, positions)
+    _require_cuda(q, layout.k, layout.v, positions, new_lens, out)
     _check_lastdim("q", q, 4)
     B, Hq, T, D = q.shape
     if D != layout.head_dim:
