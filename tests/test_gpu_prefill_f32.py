@@ -70,15 +70,37 @@ def test_two_blocks_per_workgroup():
     assert torch.allclose(torch.from_numpy(got), rows.cpu(), rtol=1e-4, atol=1e-5)
 
 
-def test_infinite_value_of_a_later_token_stays_there():
-    # value row 20 is inf: token 20 and later see it, earlier ones (same tile) must not
-    def edit(kv, values):
-        off = 20 * 64
-        kv.v[off:off + 64] = float("inf")
+@pytest.mark.parametrize("Hq,Hkv,D,paged,batch,cached", [
+    (4, 1, 64, False, 1, 0),
+    (4, 1, 128, False, 1, 0),      # width 128
+    (3, 1, 100, True, 2, 37),      # padded to 128, page pool, a prefix
+    (2, 2, 20, True, 1, 5),        # padded to 32, G 1: sixteen tokens a block
+    (32, 8, 32, False, 8, 0),      # two column blocks per workgroup
+    (32, 8, 64, True, 8, 3),
+])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_non_finite_value_of_a_later_token_stays_there(Hq, Hkv, D, paged, batch, cached, value):
+    # value row `token` of each chunk is inf or NaN: it and later tokens see it, earlier ones (same tile, same
+    # block of columns) must not
+    new = 136 if batch == 8 else 40
+    token = new - 20
 
-    got, ref, _ = _run([0], [40], 4, 1, 64, False, seed=3, edit=edit)
-    _check(got[:, :20], [r[:20] for r in ref], [20])
-    assert np.all(np.isinf(got[0, 20:]))
+    def edit(kv, values):
+        v = kv.v.view(-1)
+        for b in range(batch):
+            t = cached + token
+            if paged:
+                page = int(kv.page_table[b, t // kv.page_size])
+                row = page * kv.strides[1] + t % kv.page_size * D
+            else:
+                row = b * kv.strides[0] + t * D
+            for h in range(Hkv):
+                v[row + h * kv.strides[2]:][:D] = value
+
+    got, ref, _ = _run([cached] * batch, [new] * batch, Hq, Hkv, D, paged, seed=3, edit=edit)
+    _check(got[:, :token], [r[:token] for r in ref], [token] * batch)
+    later = got[:, token:]
+    assert np.all(np.isinf(later) if np.isinf(value) else np.isnan(later))
 
 
 def _layer(B, Hkv, D, cap, seed):

@@ -16,13 +16,18 @@
 //                  V[key 4 g + r][64 j + 4 m ..], element c being row m of the
 //                  output block with d = 64 j + 4 m + c. P needs no shuffle.
 // K's registers are reloaded for the next tile once Q K^T has used them (the
-// softmax and P V hide it), V's after P V.
+// softmax and P V hide it), V's after P V. Tiles below the workgroup's first
+// token's limit run in a loop without masks and without scratch accesses;
+// the others in one of their own.
 //
-// Bound: the fp32 matrix rate (64 flop per cycle and SIMD) and, in small
-// batches, the key walk of the longest column. Against one VALU workgroup per
-// query row, which read the whole K/V prefix per row (4 prompts U[128, 1024],
-// 8 / 2 heads, D 64; 1.0 GFLOP): 1296 + 13 us (its merge) -> 79 us.
+// Bound: in small batches the key walk of the longest column, a quarter of its
+// tiles per wave one after the other (the fp32 matrix rate, 64 flop per cycle
+// and SIMD, alone would allow a fifth of the time). Against one VALU workgroup
+// per query row, which reads the whole K/V prefix per row (4 prompts of 579,
+// 579, 828 and 226 tokens, 8 / 2 heads, D 64; 1.0 GFLOP): 1296 + 13 us (its
+// merge) -> 42 us; 76 us while the scores and O lay in scratch memory.
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_tiles.h"
 #include "tt_internal.h"
@@ -90,27 +95,30 @@ __device__ __forceinline__ bool any_nonfinite(const BlockF32<D> (&x)[2]) {
 
 // P V of one tile key by key, for a tile that some columns see only in part
 // and whose V holds an infinity or NaN: a masked key's P is 0, and 0 times
-// those would reach columns that do not attend to the key.
-template <int NO>
-__device__ __noinline__ void pv_masked(const PrefillArgs &a, const int64_t (&e)[2], int t0, int lim, int hd, int lane,
-                                       const f32x4 (&S)[2], f32x4 (&o)[NO]) {
-  const float *v = static_cast<const float *>(a.v_cache);
-  const int n = lane & 15, g = lane >> 4;
+// those would reach columns that do not attend to the key. Each step's product
+// runs once per key slot, with the other three slots' V zero, and a column
+// keeps it where it sees the key. Inlined, so that O and S stay in registers.
+template <int D, int NB, int NO>
+__device__ __forceinline__ void pv_masked(const BlockF32<D> (&x)[2], const f32x4 (&S)[NB][2], int t0, int lane,
+                                          const int (&lim)[NB], f32x4 (&o)[NB][NO]) {
+#pragma unroll 1
+  for (int slot = 0; slot < 4; ++slot)
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      for (int gk = 0; gk < 4; ++gk) {
-        const int key = 16 * h + 4 * gk + r;
-        const float p = __shfl(S[h][r], n + 16 * gk, 64);
-        if (t0 + key >= lim) continue;
+      for (int r = 0; r < 4; ++r) {
+        const int key = t0 + 16 * h + 4 * slot + r;
 #pragma unroll
-        for (int c = 0; c < NO; ++c)
+        for (int c = 0; c < NO; ++c) {
+          const float v = (lane >> 4) == slot ? x[h].v[r][c >> 2][c & 3] : 0.f;
 #pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const int d = 64 * (c >> 2) + 4 * (4 * g + w) + (c & 3);
-            if (d < hd) o[c][w] += p * v[e[h] + (int64_t)(4 * gk + r) * hd + d];
+          for (int j = 0; j < NB; ++j) {
+            const f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[j][h][r], o[j][c], 0, 0, 0);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) o[j][c][w] = key < lim[j] ? sum[w] : o[j][c][w];
           }
+          __builtin_amdgcn_sched_barrier(0);  // one block's sums in registers at a time (width 128 has none to spare)
+        }
       }
 }
 
@@ -137,7 +145,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_f32_kernel(PrefillArgs
   const int t_end = min(t_first + wg_tokens, nb);
   const int L = t_first < nb && pos0 >= 0 ? __builtin_amdgcn_readfirstlane(min(pos0 + t_end, a.max_len)) : 0;
 
-  const int lim_min = pos0 + t_first + 1;  // tiles below it are whole for every column
+  const int lim_min = min(pos0 + t_first + 1, L);  // tiles below it are whole for every column
   int lim[NB];
   float qf[NB][D / 4];
 #pragma unroll
@@ -189,7 +197,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_f32_kernel(PrefillArgs
     for (int h = 0; h < 2; ++h) load_k<D, kPad>(a, e[h], rows[h], lane, x[h]);
 #pragma unroll
     for (int h = 0; h < 2; ++h) load_v<D, kPad>(a, e[h], rows[h], lane, x[h]);
-    for (int it = c0 + wave; it < c1; it += kWaves) {
+    // One tile. A tile that some column may see only in part (kEdge) has code of its own: the masks and the
+    // registers of the key-by-key path stay out of the others'.
+    auto step = [&](int it, auto edge_tile) {
+      constexpr bool kEdge = decltype(edge_tile)::value;
       f32x4 S[NB][2];
 #pragma unroll
       for (int j = 0; j < NB; ++j)
@@ -204,7 +215,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_f32_kernel(PrefillArgs
 #pragma unroll
             for (int j = 0; j < NB; ++j)
               S[j][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[h].k[u][i], qf[j][4 * u + i], S[j][h], 0, 0, 0);
-      const int64_t ev[2] = {e[0], e[1]};
       address(min(it + kWaves, c1 - 1));  // past the span: loaded again, unused
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -218,7 +228,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_f32_kernel(PrefillArgs
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int key = kTile * it + 16 * h + 4 * g + r;
-            S[j][h][r] = key < lim[j] ? S[j][h][r] * a.scale_log2 : kNegInf;
+            S[j][h][r] = !kEdge || key < lim[j] ? S[j][h][r] * a.scale_log2 : kNegInf;
             mx = fmaxf(mx, S[j][h][r]);
           }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -239,25 +249,27 @@ __global__ __launch_bounds__(64 * kWaves, 2) void prefill_f32_kernel(PrefillArgs
 #pragma unroll
         for (int c = 0; c < NO; ++c) o[j][c] *= alpha;
       }
-      if (kTile * (it + 1) > lim_min && any_nonfinite<D>(x)) {  // uniform; see pv_masked
-#pragma unroll
-        for (int j = 0; j < NB; ++j) pv_masked<NO>(a, ev, kTile * it, lim[j], hd, lane, S[j], o[j]);
+      if (kEdge && any_nonfinite<D>(x)) {  // uniform; see pv_masked
+        pv_masked<D, NB, NO>(x, S, kTile * it, lane, lim, o);
       } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+          for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int c = 0; c < NO; ++c)
+            for (int c = 0; c < NO; ++c)
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
-              o[j][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[h].v[r][c >> 2][c & 3], S[j][h][r], o[j][c], 0, 0, 0);
+              for (int j = 0; j < NB; ++j)
+                o[j][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[h].v[r][c >> 2][c & 3], S[j][h][r], o[j][c], 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int h = 0; h < 2; ++h) load_v<D, kPad>(a, e[h], rows[h], lane, x[h]);
       __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    int it = c0 + wave;
+    for (const int whole = min(lim_min / kTile, c1); it < whole; it += kWaves) step(it, std::false_type{});
+    for (; it < c1; it += kWaves) step(it, std::true_type{});
   }
 
 #pragma unroll
