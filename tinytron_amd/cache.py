@@ -257,9 +257,10 @@ class _LayerCacheBase:
         cache; returns [B, T, H_q, D]. bf16 activations over a bf16 / fp8 cache
         whose rows are whole 16-byte fragments take the prefill kernel (rows
         past new_lens[b] untouched), fp32 over such an fp32 cache its fp32
-        counterpart; the other head dims and the fp32 forms that kernel does
-        not take (ops.prefill_f32_takes) take row attention, one query row per
-        new token (``kernel=False`` takes it for every case). fp32 and row
+        counterpart; the other head dims, the fp32 forms that kernel does not
+        take (ops.prefill_f32_takes) and a few fp32 tokens after a long prefix
+        (ops.prefill_f32_few_rows) take row attention, one query row per new
+        token (``kernel=False`` takes it for every case). fp32 and row
         attention leave zeros in the rows past new_lens[b]."""
         lay = self.layout
         T = q_rot.shape[2]
@@ -272,7 +273,9 @@ class _LayerCacheBase:
         adds = [min(int(n), T) for n in new_lens]
         cached = [x - a for x, a in zip(self._host_lens, adds)]
         if kernel and q_rot.dtype == torch.float32 and ops.prefill_f32_supported(lay, q_rot.shape[1]) \
-                and ops.prefill_f32_takes(q_rot, out, len(cached)) and min(cached, default=0) >= 0:
+                and ops.prefill_f32_takes(q_rot, out, len(cached)) and min(cached, default=0) >= 0 \
+                and not ops.prefill_f32_few_rows(sum(adds) * q_rot.shape[1], q_rot.shape[1] // lay.num_heads,
+                                                 lay.head_dim, self.current_length):
             # from the host's lengths, as row attention: the other length buffer holds those before the last
             # append only (not after set_lengths, nor for a chunk that two appends wrote)
             pos, nl = torch.tensor([cached, adds], dtype=torch.int32).to(q_rot.device, non_blocking=True)

@@ -172,7 +172,8 @@ class Attention(nn.Module):
             y = ops.decode_attention(q_rot.view(B, Hq, D), store.layout, pos + 1, t_past + 1).view(B, 1, self.n_embd)
         elif self.prefill_kernel and act == torch.bfloat16 and ops.attention_tile_dim(D, store.layout.kind):
             y = ops.prefill_attention(q_rot, store.layout, pos, t_past + T).view(B, T, self.n_embd)
-        elif self.prefill_kernel and act == torch.float32 and ops.prefill_f32_supported(store.layout, Hq):
+        elif self.prefill_kernel and act == torch.float32 and ops.prefill_f32_supported(store.layout, Hq) \
+                and not ops.prefill_f32_few_rows(B * T * Hq, 1, D, t_past + T):
             y = ops.prefill_attention_f32(q_rot, store.layout, pos, t_past + T).view(B, T, self.n_embd)
         else:
             y = ops.prefill_attention_rows(q_rot, store.layout, [t_past] * B, [T] * B).view(B, T, self.n_embd)

@@ -791,6 +791,34 @@ def prefill_f32_takes(q: torch.Tensor, out: torch.Tensor | None, num_seqs: int) 
                            and out.device == q.device)
 
 
+def prefill_f32_few_rows(columns: int, group: int, head_dim: int, max_len: int) -> bool:
+    """Whether row attention is the faster one for an fp32 chunk of ``columns``
+    = B * T * H_q (token, head) rows attending to up to ``max_len`` keys in
+    groups of ``group`` heads. The fp32 prefill kernel walks a column's whole
+    prefix in one workgroup; row attention cuts it over the GPU but reads it
+    once per row. So: few columns after a long prefix. Measured, calls of
+    prefill_attend, prefill kernel over row attention (host time counts: row
+    attention makes about 25 us of it more):
+
+      columns, heads   D    L 2048  4096  8192  16384  32768
+      8, 4 / 4        32     0.55   0.90  1.58   1.99   1.80
+      16, 8 / 8       64     0.67   1.10  1.37   1.19   1.41
+      16, 8 / 8      128     1.00   1.29  1.62   1.31   1.20
+      16, 8 / 2       64     0.47   0.71  1.08   1.43   1.62
+      16, 8 / 2      128     0.53   0.85  1.35   1.40   1.69
+      24, 12 / 4      64     0.55   0.83  1.11   1.25   0.94
+      24, 12 / 4     128     0.64   1.01  1.19   1.31   1.00
+      32, 16 / 4      32     0.47   0.68  0.93   1.17   1.06
+      32, 16 / 4      64     0.47   0.70  0.95   1.07   0.75
+      48, 16 / 4      32     0.47   0.62  0.84   0.85   0.89
+      48, 8 / 8      128     0.85   0.65  0.65   0.64   0.67"""
+    if group > 1:
+        far = 6144
+    else:
+        far = 4096 if head_dim <= 64 else 2048
+    return columns <= (32 if head_dim <= 32 else 24) and max_len >= far
+
+
 def prefill_attention_f32(q: torch.Tensor, layout: KVLayout, positions: torch.Tensor, max_seq_len: int,
                           new_lens: torch.Tensor | None = None, out: torch.Tensor | None = None,
                           sm_scale: float | None = None) -> torch.Tensor:
