@@ -1,6 +1,6 @@
 """GPU parity: merging the balanced partition's pieces, at the edges of the
-dispatch between the wide merge (at most 256 (sequence, KV head) segments) and
-the one-wave merge, and of the wide merge's own splits: one piece, fewer pieces
+dispatch between the wide merge (few (sequence, KV head) segments of many
+tiles) and the one-wave merge, and of the wide merge's own splits: one piece, fewer pieces
 than its four waves, one past a wave's 16-row batch, more than 64 pieces a wave
 (a lane each), sequences with nothing cached, every tile width and group size;
 NaN and infinite scores on both sides of the dispatch.
@@ -26,8 +26,18 @@ pytestmark = pytest.mark.gpu
     ([33000], 3, 1, 64, {}),                                # W >= NW: every wave holds a piece, G 3
     ([8000, 1, 300], 10, 2, 32, {}),                        # 32-wide rows, G 5
     ([700, 33, 1200], 8, 4, 96, dict(fp8=True, paged=True)),
-    ([40] * 32, 16, 8, 64, dict(zero_first=True)),          # 256 segments: the last the wide merge takes
-    ([40] * 33, 16, 8, 64, dict(zero_first=True)),          # 264: the one-wave merge
+    ([40] * 32, 16, 8, 64, dict(zero_first=True)),          # 256 short segments: the one-wave merge
+    ([40] * 33, 16, 8, 64, dict(zero_first=True)),          # 264: always that one
+    ([65] * 32, 8, 8, 64, {}),                              # G 1: three tiles take the wide merge,
+    ([64] * 4, 8, 8, 64, {}),                               # two the one-wave merge
+    ([64] * 17, 24, 8, 64, {}),                             # 136 segments, G 3: the wide at up to two tiles,
+    ([128] * 17, 24, 8, 64, {}),                            # the one-wave merge at three and four,
+    ([129] * 24, 24, 8, 64, {}),                            # the wide again from five on
+    ([64] * 17, 16, 8, 64, {}),                             # G 2: the one-wave merge at up to two tiles,
+    ([65] * 24, 16, 8, 128, {}),                            # the wide from three on
+    ([384] * 32, 16, 8, 64, {}),                            # 256: up to twelve tiles the one-wave merge,
+    ([385] * 32, 16, 8, 64, {}),                            # thirteen the wide, except
+    ([385] * 32, 16, 8, 128, {}),                           # on 128-wide tiles
 ])
 def test_merge_edges(lengths, Hq, Hkv, D, kw):
     got, ref, _ = run_case(lengths, Hq=Hq, Hkv=Hkv, D=D, seed=len(lengths) + D, **kw)
@@ -38,7 +48,7 @@ def test_merge_edges(lengths, Hq, Hkv, D, kw):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
-@pytest.mark.parametrize("batch", [32, 33])  # 256 and 264 segments: the wide and the one-wave merge
+@pytest.mark.parametrize("batch", [16, 32, 33])  # 128 segments: the wide merge; 264: the one-wave; 256: by length
 @pytest.mark.parametrize("lengths", [40, 700])
 def test_nan_and_infinite_scores_stay(D, batch, lengths):
     # A NaN in q, a NaN in a cached key, an infinite score: NaN rows as softmax gives them, not zeros; a score

@@ -1502,10 +1502,33 @@ hipError_t launch_mfma(const DecodeArgs &a, dim3 block, size_t lds_merge, hipStr
   return hipGetLastError();
 }
 
-// Segments up to which the wide merge runs: its segments x G workgroups of
-// four waves win while a segment has more pieces than the one-wave merge loads
-// in a round trip or two (both sides measured at decode_merge_wide_kernel).
-constexpr int64_t kMergeWideSegs = 256;
+// Whether the four-wave merge is the faster one: its segments x G workgroups
+// win while a segment's pieces are more than the one-wave merge loads in a
+// round trip or two and the workgroups do not queue for the CUs. `tiles` bounds
+// the longest segment's 32-token tiles, and so its pieces. Measured, decode
+// calls (H_kv 8, even lengths), four-wave over one-wave merge:
+//             tokens   16    64    100   200   400   800
+//   segments  G  D
+//        32   1  128  1.02  1.01  0.99  1.00  0.93  0.82
+//       128   1  128  1.02  1.02  0.99  1.00  0.98  0.98
+//       128   4  128  0.96  0.95  0.97  0.94  0.92  0.93
+//       128  16   64  0.83  0.82  0.89  0.79  0.75  0.67
+//       192   2   64  1.01  1.00  0.98  0.97  0.93  0.94
+//       192   4   64  0.96  0.95  1.00  0.99  0.93  0.93
+//       192  16   64  0.95  0.95  1.07  0.93  0.84  0.83
+//       256   1   64  1.01  1.01  0.98  0.99  0.97  0.98
+//       256   4   64  1.00  0.99  1.04  1.02  0.99  0.98
+//       256   8   64  1.03  1.02  1.12  1.01  0.99  0.97
+//       256   4  128  1.00  0.99  1.05  1.02  1.01  1.01
+//       256  16  128  0.98  0.98  1.13  1.05  0.99  0.99
+// With G 1 a workgroup per head saves nothing but the walk: three tiles or more.
+inline bool wide_merge(int64_t segs, int group, int tiles, int D) {
+  if (segs > 256) return false;
+  if (group == 1) return tiles > 2;
+  if (segs <= 128) return true;
+  if (segs <= 192) return tiles > 4 || (tiles > 2 ? group == 2 : group > 2);
+  return D < 128 && tiles > 12;
+}
 
 template <int D, bool kFP8, bool kPad>
 hipError_t launch_stream(const DecodeArgs &a0, const DecodeAppend *ap, hipStream_t stream) {
@@ -1533,7 +1556,7 @@ hipError_t launch_stream(const DecodeArgs &a0, const DecodeAppend *ap, hipStream
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   const int64_t segs = (int64_t)a.batch * a.hkv;
-  if (segs <= kMergeWideSegs) {
+  if (wide_merge(segs, a.group, (a.max_len + 31) / 32, D)) {
     hipLaunchKernelGGL((decode_merge_wide_kernel<D>), dim3(a.group, (unsigned)segs), dim3(64 * kWavesPerBlock), 0,
                        stream, a);
     return hipGetLastError();
