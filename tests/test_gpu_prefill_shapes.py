@@ -1,0 +1,65 @@
+"""GPU parity: every workgroup shape that prefill attention picks, on both sides
+of each line of its rule (keys within one tile or past it, columns for up to 4
+waves or more, pairs up to what the GPU holds at once or past it: 256 CUs), for
+ragged chunks over a page pool, unpadded and padded widths, 20 tokens past a
+1024-token page-entry span. Reference: row attention, a kernel of its own.
+
+Tolerance: the attention tests' bound against the exact result (2e-3 + 2e-2
+|ref|) twice over, since both sides may be that far from it.
+"""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+DTYPE = {"bf16": torch.bfloat16, "fp8": torch.float8_e4m3fn}
+
+
+def _cache(kind, B, Hkv, D, total, g):
+    from tinytron_amd.cache import PagedLayerKVCache, random_page_table
+
+    table, pages = random_page_table(total, 16, seed=B)
+    c = PagedLayerKVCache(table, pages, Hkv, D, 16, "cuda", DTYPE[kind])
+    for data, scale in ((c.layout.k, c.layout.k_scale), (c.layout.v, c.layout.v_scale)):
+        if kind == "bf16":
+            data.normal_(generator=g)
+        else:  # every finite code, scales of up to 2 / 448
+            codes = torch.randint(0, 254, data.shape, generator=g, device="cuda", dtype=torch.int16)
+            data.copy_((codes + (codes >= 127)).to(torch.uint8))
+            scale.copy_(torch.rand(scale.shape, generator=g, device="cuda") / 224)
+    return c
+
+
+@pytest.mark.parametrize("kind,D,G,Hkv,B,past,new", [
+    # bf16, width 32: 8 x 64 to 512 pairs, 4 x 32 past them, 2 x 32 past 1024 with columns for two waves
+    ("bf16", 32, 4, 8, 64, 70, 9), ("bf16", 32, 4, 8, 65, 70, 9), ("bf16", 24, 4, 8, 129, 70, 16),
+    ("bf16", 32, 4, 8, 129, 70, 17), ("bf16", 32, 4, 8, 129, 70, 33), ("bf16", 32, 1, 16, 65, 3, 61),
+    # width 64
+    ("bf16", 64, 4, 8, 64, 70, 9), ("bf16", 64, 4, 8, 65, 70, 32), ("bf16", 40, 4, 8, 65, 70, 33),
+    ("bf16", 64, 8, 2, 3, 4, 60), ("bf16", 48, 8, 2, 3, 5, 60),
+    # width 128: 256 pairs
+    ("bf16", 128, 4, 8, 32, 70, 9), ("bf16", 128, 4, 8, 33, 70, 32), ("bf16", 96, 3, 8, 33, 70, 41),
+    ("bf16", 128, 16, 1, 2, 0, 64), ("bf16", 128, 16, 1, 2, 1, 64),
+    # fp8, width 64: 768 pairs
+    ("fp8", 64, 4, 16, 48, 70, 9), ("fp8", 64, 4, 16, 49, 70, 32), ("fp8", 48, 4, 16, 49, 70, 33),
+    ("fp8", 64, 8, 2, 3, 4, 60),
+    # fp8, width 128: a wave per pair for up to 64 keys or one wave's columns past 512 pairs; 4 x 64; 8 x 64
+    ("fp8", 128, 4, 8, 2, 32, 32), ("fp8", 128, 4, 8, 2, 33, 32), ("fp8", 96, 6, 2, 3, 40, 20),
+    ("fp8", 128, 4, 8, 65, 1200, 8), ("fp8", 96, 4, 8, 65, 500, 7), ("fp8", 128, 4, 8, 64, 70, 8),
+    ("fp8", 128, 4, 8, 32, 70, 30), ("fp8", 128, 4, 8, 33, 70, 30), ("fp8", 80, 5, 4, 65, 70, 21),
+    ("fp8", 128, 4, 2, 5, 1030, 150), ("fp8", 128, 4, 8, 17, 300, 100), ("fp8", 128, 4, 8, 17, 500, 100),
+])
+def test_shapes_against_row_attention(kind, D, G, Hkv, B, past, new):
+    from tinytron_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(B + D + new)
+    pick = torch.Generator().manual_seed(B)
+    cached = [past] + torch.randint(0, past + 1, (B - 1,), generator=pick).tolist()
+    news = [new] + torch.randint(0, new + 1, (B - 1,), generator=pick).tolist()
+    c = _cache(kind, B, Hkv, D, [o + n for o, n in zip(cached, news)], g)
+    q = torch.randn(B, Hkv * G, new, D, generator=g, device="cuda").bfloat16()
+    out = torch.zeros(B, new, Hkv * G, D, device="cuda", dtype=torch.bfloat16)
+    ops.prefill_attention(q, c.layout, torch.tensor(cached, dtype=torch.int32, device="cuda"), past + new,
+                          new_lens=torch.tensor(news, dtype=torch.int32, device="cuda"), out=out)
+    ref = ops.prefill_attention_rows(q, c.layout, cached, news).float()
+    assert ((out.float() - ref).abs() <= 2 * (2e-3 + 2e-2 * ref.abs())).all()

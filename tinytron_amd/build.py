@@ -17,8 +17,8 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libtinytron_amd.so"
 OBJ_DIR = PKG_DIR / "_build"  # per-source objects (git-ignored)
-SOURCES = ["abi.hip", "rope_append.hip", "decode_attn.hip", "prefill_attn.hip", "prefill_attn_f32.hip",
-           "layer_ops.hip", "sampler.hip"]
+SOURCES = ["abi.hip", "rope_append.hip", "decode_attn.hip", "prefill_attn.hip", "prefill_attn_stream.hip",
+           "prefill_attn_f32.hip", "layer_ops.hip", "sampler.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

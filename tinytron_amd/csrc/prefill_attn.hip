@@ -66,24 +66,26 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Waves per workgroup (32 columns each) and the waves per SIMD that the
-// registers must leave room for. bf16 at tile width <= 64 fits 128 registers: two
-// workgroups of 8 waves per CU. Width 128 (q and O alone take 96 registers)
-// runs one; fp8 at width 64 (the scales' registers) three of 4 waves. Wider
-// workgroups read the pair's K/V from L2 less often; more waves per SIMD run
+// Waves per workgroup (32 columns each), keys per LDS tile and the waves per SIMD
+// that the registers must leave room for. bf16 at tile width <= 64 fits 128
+// registers: two workgroups of 8 waves per CU. Width 128 (q and O alone take 96
+// registers) runs one; fp8 at width 64 (the scales' registers) three of 4 waves.
+// Wider workgroups read the pair's K/V from L2 less often; more waves per SIMD run
 // one's softmax beside another's MFMAs. Measured (C5 prompts, D 64): 8 waves x
 // two workgroups 717 us, two 32-column blocks a wave at two waves per SIMD 750,
 // 4 waves x three 786; (prefix 2k-8k, fp8, D 128): 8 waves 1154-1190 us, 4
-// waves x two 1171-1292, tiles of 128 keys 1289.
-template <int D, bool kFP8>
+// waves x two 1171-1292, tiles of 128 keys 1289. Which shape runs: launch_d.
+template <int kD, bool kIsFP8, int kWaves, int kTileKeys>
 struct PrefillShape {
-  static constexpr int NW = D == 64 && kFP8 ? 4 : 8;
+  static constexpr int D = kD;
+  static constexpr bool kFP8 = kIsFP8;
+  static constexpr int NW = kWaves;
   static constexpr int kOcc = D == 128 ? 2 : D == 64 && kFP8 ? 3 : 4;
-  static constexpr int kKeys = 64;  // keys per LDS tile
+  static constexpr int kKeys = kTileKeys;  // keys per LDS tile
   static constexpr int kThreads = 64 * NW;
   static constexpr int kRowBytes = 2 * D;           // LDS rows hold bf16
   static constexpr int kTileBytes = kKeys * kRowBytes;
-  // LDS: K[2] | V[2] | fp8: K scales [2][64], V scales [2][64]
+  // LDS: K[2] | V[2] | fp8: K scales [2][kKeys], V scales [2][kKeys]
   static constexpr int kScaleAt = 4 * kTileBytes;
   static constexpr int kLds = kScaleAt + (kFP8 ? 4 * kKeys * 4 : 0);
 };
@@ -102,10 +104,9 @@ __device__ __forceinline__ int v_swizzle(int r) {
 
 // This thread's share of one tile on its way from the cache to LDS: N of the
 // tile's 16-byte chunks, K's rows first, then V's.
-template <int D, bool kFP8>
+template <class SH>
 struct Staged {
-  using SH = PrefillShape<D, kFP8>;
-  static constexpr int kChunks = D * (kFP8 ? 1 : 2) / 16;  // of a cached row
+  static constexpr int kChunks = SH::D * (SH::kFP8 ? 1 : 2) / 16;  // of a cached row
   static constexpr int kHalf = SH::kKeys * kChunks;        // K's chunks
   static constexpr int N = 2 * kHalf / SH::kThreads;
   static_assert(N * SH::kThreads == 2 * kHalf && kHalf % 64 == 0 && 64 / kChunks <= 16, "a wave: K or V, one block");
@@ -123,10 +124,12 @@ struct Staged {
 // Issue the loads of the tile at key t0. `entry` holds, one per lane, the
 // page-table entries of pages pbase.. (see stream_block_addr); rows past L and
 // chunks past a padded row's end read zero (the buffer range).
-template <int D, bool kFP8, bool kPad>
+template <class SH, bool kPad>
 __device__ __forceinline__ void stage_load(const DecodeArgs &a, int b, int hk, int L, int entry, int pbase, int t0,
-                                           Staged<D, kFP8> &st) {
-  using ST = Staged<D, kFP8>;
+                                           Staged<SH> &st) {
+  using ST = Staged<SH>;
+  constexpr int D = SH::D;
+  constexpr bool kFP8 = SH::kFP8;
   constexpr int E = KVTraits<kFP8>::kElemBytes;
   const int hd = row_len<D, kPad>(a);
   const int c = ST::chunk();
@@ -151,10 +154,11 @@ __device__ __forceinline__ void stage_load(const DecodeArgs &a, int b, int hk, i
 }
 
 // The staged pieces into LDS buffer `buf` as bf16 rows.
-template <int D, bool kFP8>
-__device__ __forceinline__ void stage_store(const DecodeArgs &a, const Staged<D, kFP8> &st, char *lds, int buf) {
-  using ST = Staged<D, kFP8>;
-  using SH = PrefillShape<D, kFP8>;
+template <class SH>
+__device__ __forceinline__ void stage_store(const DecodeArgs &a, const Staged<SH> &st, char *lds, int buf) {
+  using ST = Staged<SH>;
+  constexpr int D = SH::D;
+  constexpr bool kFP8 = SH::kFP8;
   const int c = ST::chunk();
 #pragma unroll
   for (int j = 0; j < ST::N; ++j) {
@@ -196,9 +200,10 @@ __device__ __forceinline__ void split_p(const float (&p)[8], bf16x8 &hi, bf16x8 
   lo = __builtin_convertvector(rem, bf16x8);
 }
 
-template <int D, bool kFP8, bool kPad>
-__global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D, kFP8>::kOcc)) void prefill_attn_kernel(PrefillArgs a) {
-  using SH = PrefillShape<D, kFP8>;
+template <class SH, bool kPad>
+__global__ __launch_bounds__(SH::kThreads, SH::kOcc) void prefill_attn_kernel(PrefillArgs a) {
+  constexpr int D = SH::D;
+  constexpr bool kFP8 = SH::kFP8;
   constexpr int kKeys = SH::kKeys;
   constexpr int NU = kKeys / 32;
   const auto mx2 = [](float u, float v) { return __builtin_elementwise_maximum(u, v); };
@@ -260,10 +265,10 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
       entry = a.page_table[(int64_t)b * a.max_pages + min(pbase + lane, last_page)];
     }
   };
-  Staged<D, kFP8> st;
+  Staged<SH> st;
   fetch_entries(0);
-  stage_load<D, kFP8, kPad>(a, b, hk, L, entry, pbase, 0, st);
-  stage_store<D, kFP8>(a, st, lds, 0);
+  stage_load<SH, kPad>(a, b, hk, L, entry, pbase, 0, st);
+  stage_store<SH>(a, st, lds, 0);
   __syncthreads();
 
   // this lane's K row and V rows (see k_swizzle / v_swizzle); XORed with the
@@ -285,7 +290,7 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
     const bool more = i + 1 < tiles;
     if (more) {
       if ((kKeys * (i + 1)) % 1024 == 0) fetch_entries(i + 1);
-      stage_load<D, kFP8, kPad>(a, b, hk, L, entry, pbase, kKeys * (i + 1), st);
+      stage_load<SH, kPad>(a, b, hk, L, entry, pbase, kKeys * (i + 1), st);
     }
     __builtin_amdgcn_sched_barrier(0);
     const char *kb = lds + (i & 1) * SH::kTileBytes;
@@ -302,7 +307,7 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
       for (int u = 0; u < NU; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) S[u][r] = 0.f;
-      if (!kEdge || Lw - t0 > 32) {  // uniform
+      if (NU == 1 || !kEdge || Lw - t0 > 32) {  // uniform
 #pragma unroll
         for (int s = 0; s < D / 16; ++s)
 #pragma unroll
@@ -408,7 +413,7 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
     }
     __builtin_amdgcn_sched_barrier(0);
     // the other buffer's readers are done since the last barrier
-    if (more) stage_store<D, kFP8>(a, st, lds, (i + 1) & 1);
+    if (more) stage_store<SH>(a, st, lds, (i + 1) & 1);
     __syncthreads();
   };
   int i = 0;
@@ -445,16 +450,63 @@ __global__ __launch_bounds__((PrefillShape<D, kFP8>::kThreads), (PrefillShape<D,
     }
 }
 
-template <int D, bool kFP8, bool kPad>
-hipError_t launch_d(const PrefillArgs &a0, hipStream_t stream) {
-  using SH = PrefillShape<D, kFP8>;
-  PrefillArgs a = a0;
+template <class SH, bool kPad>
+hipError_t launch_shape(PrefillArgs a, hipStream_t stream) {
   a.qt = 32 / a.group;  // group <= 16
   const int wg_tokens = a.qt * SH::NW;
   a.wg_per_pair = (a.num_new + wg_tokens - 1) / wg_tokens;
-  hipLaunchKernelGGL((prefill_attn_kernel<D, kFP8, kPad>), dim3((unsigned)prefill_grid(a)), dim3(SH::kThreads), 0, stream,
-                     a);
+  hipLaunchKernelGGL((prefill_attn_kernel<SH, kPad>), dim3((unsigned)prefill_grid(a)), dim3(SH::kThreads), 0, stream, a);
   return hipGetLastError();
+}
+
+// Which workgroup runs a call. Wide ones (64-key tiles; 8 waves, fp8 at width
+// 64: 4) stage a pair's K/V once for many columns and hide its latency best, but
+// they hold all their waves, LDS and registers also where a pair's columns fill
+// few of the waves, and for a few keys one 64-key tile is a long chain. So with
+// keys within one tile, or columns for at most 4 waves on more pairs than the GPU
+// holds wide workgroups: 4 waves on 32-key tiles (at width 32 and columns for two
+// waves, on twice as many pairs, 2 waves), of which a CU holds two to four times
+// as many. fp8 at width 128, whose registers allow 8 waves a CU in any case:
+//  * up to 4 waves of columns: a wave per pair streaming K/V for itself
+//    (prefill_attn_stream.hip) for keys within one tile, and for one wave of
+//    columns once two 4-wave workgroups a CU do not hold the pairs; 4 waves on
+//    64-key tiles past a pair per CU; 8 waves below, whose staging is the fastest;
+//  * more columns: 4 waves where that fills idle CUs or keys are few, 8 otherwise.
+// Measured, us (G 4, T new tokens after P cached; pairs of (sequence, KV head)):
+//             D   pairs     P    T   wide  chosen
+//   bf16     32    2048     0    2   12.5     4.9   2 x 32
+//   bf16     32    2048  1000    8   67.8    44.4   2 x 32
+//   bf16     64     512     0    8    5.6     4.3   4 x 32
+//   bf16     64    1024   250    8   21.4    15.8   4 x 32
+//   bf16     64    1024  4000    8  194.0   194.3   4 x 32
+//   bf16    128     256     0   64   16.7    13.8   4 x 32
+//   bf16    128     512  1000    8   65.8    47.2   4 x 32
+//   fp8      64    1024  1000    8   59.8    36.5   4 x 32
+//   fp8     128       8     0   20    6.4     4.9   a wave each
+//   fp8     128    1024  1000    8  140.7    56.9   a wave each
+//   fp8     128     512  1000    8   69.8    46.8   4 x 64
+//   fp8     128       8  4000  200  186.1   163.8   4 x 64
+//   fp8     128     256     0  200   68.7    51.3   4 x 64
+//   fp8     128     128  1000  200  127.0   (4 x 64: 136)  8 x 64
+template <int D, bool kFP8, bool kPad>
+hipError_t launch_d(const PrefillArgs &a, hipStream_t stream) {
+  const int cus = device_cu_count();
+  const int64_t pairs = (int64_t)a.batch * a.hkv;
+  const int qt = 32 / a.group;                  // group <= 16
+  const int waves = (a.num_new + qt - 1) / qt;  // that a pair's columns fill
+  if constexpr (kFP8 && D == 128) {
+    if (waves <= 4 && (a.max_len <= 64 || (waves == 1 && pairs > 2 * cus))) return launch_prefill_attn_stream_fp8(a, stream);
+    const int64_t wg8 = pairs * ((waves + 7) / 8), wg4 = pairs * ((waves + 3) / 4);
+    if (waves <= 4 ? pairs > cus : wg4 <= cus || (a.max_len <= 512 && wg8 > cus))
+      return launch_shape<PrefillShape<D, kFP8, 4, 64>, kPad>(a, stream);
+  } else {
+    const int64_t slots = (int64_t)cus * (D == 128 ? 1 : kFP8 ? 3 : 2);  // wide workgroups that the GPU holds
+    if constexpr (D == 32)
+      if (waves <= 2 && pairs > 2 * slots) return launch_shape<PrefillShape<D, kFP8, 2, 32>, kPad>(a, stream);
+    if (a.max_len <= 64 || (waves <= 4 && pairs > slots))
+      return launch_shape<PrefillShape<D, kFP8, 4, 32>, kPad>(a, stream);
+  }
+  return launch_shape<PrefillShape<D, kFP8, kFP8 && D == 64 ? 4 : 8, 64>, kPad>(a, stream);
 }
 
 }  // namespace

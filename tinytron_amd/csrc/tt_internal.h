@@ -186,6 +186,8 @@ struct PrefillArgs : DecodeArgs {
 };
 
 hipError_t launch_prefill_attn(const PrefillArgs &a, CacheKind kind, int head_dim, hipStream_t stream);
+// fp8 caches of head_dim 65 .. 128, a wave per pair (launch_prefill_attn's choice for many pairs of few tokens)
+hipError_t launch_prefill_attn_stream_fp8(PrefillArgs a, hipStream_t stream);
 // fp32 caches: whole 16-byte fragments (head_dim a multiple of 4, <= 128); rows past new_lens are zeroed
 bool prefill_f32_supported(int64_t head_dim);
 hipError_t launch_prefill_attn_f32(const PrefillArgs &a, int head_dim, hipStream_t stream);
