@@ -63,3 +63,20 @@ def test_shapes_against_row_attention(kind, D, G, Hkv, B, past, new):
                           new_lens=torch.tensor(news, dtype=torch.int32, device="cuda"), out=out)
     ref = ops.prefill_attention_rows(q, c.layout, cached, news).float()
     assert ((out.float() - ref).abs() <= 2 * (2e-3 + 2e-2 * ref.abs())).all()
+
+
+def test_more_workgroups_than_one_launch_holds():
+    # 2^24 + 5 sequences of one token (256 threads each: past 2^32), all on the one page of four cached tokens
+    from tinytron_amd import ops
+
+    B, D = 2 ** 24 + 5, 8
+    g = torch.Generator(device="cuda").manual_seed(1)
+    k, v = (torch.randn(16, D, generator=g, device="cuda").bfloat16() for _ in "kv")
+    kv = ops.KVLayout(k=k.view(-1), v=v.view(-1), strides=(0, 16 * D, 16 * D), num_heads=1, head_dim=D, page_size=16,
+                      capacity=16, kind="bf16", page_table=torch.zeros(B, 1, dtype=torch.int32, device="cuda"), num_pages=1)
+    q = torch.randn(B, 1, 1, D, generator=g, device="cuda").bfloat16()
+    got = ops.prefill_attention(q, kv, torch.full((B,), 3, dtype=torch.int32, device="cuda"), 4).view(B, D)
+    for rows in (slice(0, 64), slice(2 ** 24 - 40, B)):
+        scores = q.view(B, D)[rows].float() @ k[:4].float().t() / D ** 0.5
+        ref = torch.softmax(scores, -1) @ v[:4].float()
+        assert ((got[rows].float() - ref).abs() <= 2e-3 + 2e-2 * ref.abs()).all()

@@ -441,14 +441,15 @@ constexpr int kSpreadPairs = 32;
 
 __device__ __forceinline__ bool prefill_group(const PrefillArgs &a, int &pair, int &grp) {
   const int pairs = a.batch * a.hkv;
+  const int wg = a.wg_first + blockIdx.x;
   if (pairs < kSpreadPairs) {
-    const int k = blockIdx.x / pairs;
-    pair = (blockIdx.x + k) % pairs;  // rotated: a pair's groups meet every XCD
+    const int k = wg / pairs;
+    pair = (wg + k) % pairs;  // rotated: a pair's groups meet every XCD
     grp = a.wg_per_pair - 1 - k;
     return true;
   }
-  const int slot = blockIdx.x / kPrefillXcds;
-  pair = (slot / a.wg_per_pair) * kPrefillXcds + blockIdx.x % kPrefillXcds;
+  const int slot = wg / kPrefillXcds;
+  pair = (slot / a.wg_per_pair) * kPrefillXcds + wg % kPrefillXcds;
   grp = a.wg_per_pair - 1 - slot % a.wg_per_pair;
   return pair < pairs;
 }
@@ -457,6 +458,22 @@ inline int64_t prefill_grid(const PrefillArgs &a) {
   const int64_t pairs = (int64_t)a.batch * a.hkv;
   if (pairs < kSpreadPairs) return pairs * a.wg_per_pair;
   return (pairs + kPrefillXcds - 1) / kPrefillXcds * kPrefillXcds * a.wg_per_pair;
+}
+
+// All groups' workgroups of `threads` threads, by launch(grid, args): a launch
+// holds fewer than 2^32 threads (8 M workgroups of 512), so more of them go in
+// several launches, each of whole rounds over the XCDs.
+template <class Launch>
+hipError_t launch_prefill_groups(PrefillArgs a, int threads, Launch launch) {
+  const int64_t total = prefill_grid(a), step = ((((int64_t)1 << 32) - 1) / threads) & ~(int64_t)(kPrefillXcds - 1);
+  if (total > INT32_MAX) return hipErrorInvalidConfiguration;
+  for (int64_t first = 0; first < total; first += step) {
+    a.wg_first = (int)first;
+    launch(dim3((unsigned)(total - first < step ? total - first : step)), a);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
 }
 
 }  // namespace

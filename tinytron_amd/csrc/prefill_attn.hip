@@ -455,8 +455,9 @@ hipError_t launch_shape(PrefillArgs a, hipStream_t stream) {
   a.qt = 32 / a.group;  // group <= 16
   const int wg_tokens = a.qt * SH::NW;
   a.wg_per_pair = (a.num_new + wg_tokens - 1) / wg_tokens;
-  hipLaunchKernelGGL((prefill_attn_kernel<SH, kPad>), dim3((unsigned)prefill_grid(a)), dim3(SH::kThreads), 0, stream, a);
-  return hipGetLastError();
+  return launch_prefill_groups(a, SH::kThreads, [&](dim3 grid, const PrefillArgs &args) {
+    hipLaunchKernelGGL((prefill_attn_kernel<SH, kPad>), grid, dim3(SH::kThreads), 0, stream, args);
+  });
 }
 
 // Which workgroup runs a call. Wide ones (64-key tiles; 8 waves, fp8 at width

@@ -319,8 +319,9 @@ hipError_t launch_nb(PrefillArgs a, hipStream_t stream) {
   a.qt = 16 / a.group;  // group <= 16
   const int wg_tokens = a.qt * NB;
   a.wg_per_pair = (a.num_new + wg_tokens - 1) / wg_tokens;
-  hipLaunchKernelGGL((prefill_f32_kernel<D, kPad, NB>), dim3((unsigned)prefill_grid(a)), dim3(64 * kWaves), 0, stream, a);
-  return hipGetLastError();
+  return launch_prefill_groups(a, 64 * kWaves, [&](dim3 grid, const PrefillArgs &args) {
+    hipLaunchKernelGGL((prefill_f32_kernel<D, kPad, NB>), grid, dim3(64 * kWaves), 0, stream, args);
+  });
 }
 
 // Two column blocks per workgroup halve the K/V reads per product; one spreads

@@ -179,12 +179,12 @@ hipError_t launch_prefill_attn_stream_fp8(PrefillArgs a, hipStream_t stream) {
   a.qt = 16 / a.group;  // group <= 16
   const int wave_tokens = a.qt * kBlocks;
   a.wg_per_pair = (a.num_new + wave_tokens - 1) / wave_tokens;
-  const dim3 grid((unsigned)prefill_grid(a));
-  if (a.head_dim == kD)
-    hipLaunchKernelGGL((prefill_stream_kernel<false>), grid, dim3(64), 0, stream, a);
-  else
-    hipLaunchKernelGGL((prefill_stream_kernel<true>), grid, dim3(64), 0, stream, a);
-  return hipGetLastError();
+  return launch_prefill_groups(a, 64, [&](dim3 grid, const PrefillArgs &args) {
+    if (a.head_dim == kD)
+      hipLaunchKernelGGL((prefill_stream_kernel<false>), grid, dim3(64), 0, stream, args);
+    else
+      hipLaunchKernelGGL((prefill_stream_kernel<true>), grid, dim3(64), 0, stream, args);
+  });
 }
 
 }  // namespace tt

@@ -182,6 +182,7 @@ struct PrefillArgs : DecodeArgs {
   int num_new;                 // T
   int qt;                      // query tokens per block of columns (set by the launcher)
   int wg_per_pair;             // workgroups per (sequence, KV head) (set by the launcher)
+  int wg_first;                // index of the launch's first workgroup (set by the launcher)
   int vec_out;                 // out 8-byte aligned, strides multiples of 4: 4 head_dim entries per store
 };
 
