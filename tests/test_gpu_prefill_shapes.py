@@ -80,3 +80,22 @@ def test_more_workgroups_than_one_launch_holds():
         scores = q.view(B, D)[rows].float() @ k[:4].float().t() / D ** 0.5
         ref = torch.softmax(scores, -1) @ v[:4].float()
         assert ((got[rows].float() - ref).abs() <= 2e-3 + 2e-2 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("D,B,past,new", [(128, 65, 100, 8), (128, 65, 1200, 3), (80, 130, 33, 4), (128, 3, 0, 20)])
+def test_streaming_waves_repeat_themselves(D, B, past, new):
+    # fp8 at width 128, a wave per pair with counted waits: lengths of odd and even numbers of 32-token tiles and of
+    # 16-tile spans, each pass as the first one and as row attention
+    from tinytron_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(D + B)
+    pick = torch.Generator().manual_seed(past)
+    cached = [past] + torch.randint(0, past + 1, (B - 1,), generator=pick).tolist()
+    c = _cache("fp8", B, 8, D, [o + new for o in cached], g)
+    q = torch.randn(B, 32, new, D, generator=g, device="cuda").bfloat16()
+    pos = torch.tensor(cached, dtype=torch.int32, device="cuda")
+    first = ops.prefill_attention(q, c.layout, pos, past + new)
+    ref = ops.prefill_attention_rows(q, c.layout, cached, [new] * B).float()
+    assert ((first.float() - ref).abs() <= 2 * (2e-3 + 2e-2 * ref.abs())).all()
+    for _ in range(8):
+        assert torch.equal(ops.prefill_attention(q, c.layout, pos, past + new), first)
