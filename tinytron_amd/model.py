@@ -35,6 +35,7 @@ see only the sum(new_lens) real tokens, not the B x T padded grid.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import weakref
 from dataclasses import dataclass
@@ -63,6 +64,11 @@ class ModelConfig:
     init_std: float = 0.013
     tied_lm_head: bool = True
     rope_theta: float = 10000.0
+
+
+@functools.lru_cache(maxsize=None)
+def _cu_count(device: torch.device) -> int:
+    return torch.cuda.get_device_properties(device).multi_processor_count
 
 
 _ROPE_TABLES: dict = {}
@@ -309,16 +315,22 @@ class GPT(nn.Module):
         * gate|up: 1024, with half the partials, for up to 16 rows (equal
           time: K 5120, N 27648, 5 rows 54.7 us against 54.4) and for wider
           batches where one workgroup per CU takes it whole (N 12288, K 2048:
-          14.7 us against 16.1; N 27648, K 5120, 64 rows: 89 us against 72)."""
+          14.7 us against 16.1; N 27648, K 5120, 64 rows: 89 us against 72),
+          of 96 rows of weights (128, 64) where those divide N.
+
+        Whole steps of three layers of K 1280, 2560, 3840, 4096 and 5120 at 1, 5,
+        16, 17, 32 and 64 rows took 0.57 to 1.01 of their time with widths that
+        followed K alone (gate|up 1024, c_proj 256, the others 512; row tiles of 64)."""
         c = self.config
-        C, inter, cus = c.hidden_size, c.intermediate_size, 256
+        C, inter, cus = c.hidden_size, c.intermediate_size, _cu_count(self.wte.weight.device)
         qkv = self._k_chunk(C)
         if B <= 32 and C // qkv > ops.FUSED_STEP_MAX_SPLITS and C % 1280 == 0 \
                 and C // 1280 <= ops.FUSED_STEP_MAX_SPLITS:
             qkv = 1280
         o = 256 if C % 512 or 4 * (C // 128) * (C // 512) < 3 * cus else 512
         gu = self._k_chunk(C)
-        if C % 1024 == 0 and (B <= 16 or (B > 32 and (2 * inter // 96) * (C // 1024) <= cus)):
+        rows = next((w for w in (96, 128, 64) if 2 * inter % w == 0), 64)
+        if C % 1024 == 0 and (B <= 16 or (B > 32 and (2 * inter // rows) * (C // 1024) <= cus)):
             gu = 1024
         return qkv, o, gu, self._k_chunk(inter)
 
