@@ -33,7 +33,7 @@ def test_prefill_workgroup_edges(past, new, Hq, Hkv, D, kw):
 @pytest.mark.parametrize("G,D,fp8", [(4, 64, False), (1, 64, False), (16, 128, False), (3, 32, False),
                                      (4, 64, True), (8, 128, True)])
 @pytest.mark.parametrize("past,token", [(0, 40), (0, 79), (21, 33), (50, 14)])
-def test_infinite_value_of_a_later_token_stays_there(G, D, fp8, past, token):
+def test_infinite_value_stays_out_of_earlier_waves(G, D, fp8, past, token):
     # Value row `token` of a chunk of 80 is infinite (fp8: its codes NaN, its scale infinite). The tokens
     # of earlier waves (32 // G tokens each) share its 64-key tile and must not see it, bit for bit.
     from tinytron_amd import ops

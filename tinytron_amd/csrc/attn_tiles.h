@@ -435,7 +435,12 @@ __device__ __forceinline__ void stream_block_addr(const DecodeArgs &a, int b, in
 // of 32 pairs with 2k-8k cached tokens took 1511 us against 1154). Fewer pairs
 // would leave XCDs idle or give one the longest sequence whole: their groups
 // are dealt over all XCDs, longest first (fp32, 8 pairs of U[128, 1024] tokens:
-// 97.7 us with a pair per XCD, 78.6 us dealt).
+// 97.7 us with a pair per XCD, 78.6 us dealt). Round the line,
+// 126 uneven batches of 8 to 128 pairs (1, 4 and 8 KV heads, D 64 and 128, both
+// cache types) took 0.66 to 0.93 of the time of a wave per 64 columns streaming
+// K/V for itself, one 1.04 (fp8, 16 pairs), with no step at 32. What the rule
+// leaves: with 4 KV heads a pair's XCD, its number mod 8, serves every second
+// sequence, so uneven lengths load the XCDs unevenly.
 constexpr int kPrefillXcds = 8;
 constexpr int kSpreadPairs = 32;
 

@@ -7,10 +7,11 @@
 // append, get_kv, then SDPA with is_causal=True at past_len 0 or the mask
 // key_pos <= past_len + query_pos otherwise) for a ragged batch.
 //
-// One workgroup per (sequence b, KV head hk, 256 columns), a column being one
-// (query token, head of the group) pair: a wave owns 32 of them
-// (qt = 32 / G consecutive tokens) and walks the keys in tiles of 64 that
-// the whole workgroup shares through LDS. Every thread loads its 16-byte
+// One workgroup of 2, 4 or 8 waves (PrefillShape; which one: launch_d) per
+// (sequence b, KV head hk, group of columns), a column being one (query token,
+// head of the group) pair: a wave owns 32 of them (qt = 32 / G consecutive
+// tokens) and walks the keys in tiles of 64 or 32 that the whole workgroup
+// shares through LDS. Every thread loads its 16-byte
 // pieces of the next tile's K and V into registers while the current tile is
 // computed and writes them to the other LDS buffer afterwards (one barrier a
 // tile); fp8 codes become bf16 on the way (exact), once per workgroup, so the
@@ -31,6 +32,11 @@
 // wave leaves out the 32 keys of Q K^T and the 16-key steps of P V past its last
 // token and takes V past it as zero: the tile holds values of later waves'
 // tokens, and an infinity or NaN there would reach this wave's columns as 0 x inf.
+// Limit: within a wave that is what happens. An infinite or NaN value row turns
+// the outputs of the earlier tokens that share its wave (32 / G of them, counted
+// from the chunk's first) NaN in its head dim. Telling them apart takes a pass per
+// key (20 to 57 registers spilled) or a check of each edge tile's V (short prompts
+// 5-12 % slower); the fp32 kernel has it.
 //
 // Bound: the shared issue of VALU and matrix instructions. Per 32 x 32 block at
 // D 64 a wave issues ~125 VALU instructions (16 exponentials; the P split is 48,
@@ -38,13 +44,16 @@
 // SIMD take 200 ns where either alone takes 145-160, so the two overlap by
 // half. With the same shape and timing-only loads of two fixed tiles the time
 // does not move: K/V traffic does not bind. Against one wave per 64 columns
-// streaming K/V for itself (K in registers, 16x16x32 MFMAs), kernel time:
-//   C5 prompts (64 x U[64, 2048], 32 / 8 heads)  D 64   bf16  843 -> 717 us
-//                                                       fp8  1019 -> 830 us
-//   4 x U[1024, 2048] after U[2048, 8192] cached D 128  fp8  1477 -> 1175 us
-//   8 x U[64, 4096]                              D 128  bf16  741 -> 601 us
-//   1 x 20 after 8000 cached                     D 128  bf16  409 -> 228 us
-//   6 x U[64, 2048], 32 / 4 heads                D 32   bf16  103 -> 70 us
+// streaming K/V for itself (K in registers, 16x16x32 MFMAs), calls on the same
+// lengths drawn once (32 / 8 heads unless said):
+//   64 x U[64, 2048]                             D 64   bf16  825 -> 725 us
+//                                                       fp8   984 -> 797 us
+//   4 x U[1024, 2048] after U[2048, 8192] cached D 128  fp8  1212 -> 896 us
+//   8 x U[64, 4096]                              D 128  bf16  983 -> 777 us
+//   1 x 20 after 8000 cached                     D 128  bf16  394 -> 226 us
+//   6 x U[64, 2048], 32 / 4 heads                D 32   bf16   81 -> 67 us
+// The last but one is bound otherwise: 8 workgroups, each walking its pair's 8020
+// keys tile after tile, leave 248 CUs idle.
 //
 // With many pairs, all query blocks of one (sequence, KV head) run on one XCD,
 // whose L2 keeps the pair's K/V for them (prefill_group).
@@ -483,9 +492,9 @@ hipError_t launch_shape(PrefillArgs a, hipStream_t stream) {
 //   bf16    128     256     0   64   16.7    13.8   4 x 32
 //   bf16    128     512  1000    8   65.8    47.2   4 x 32
 //   fp8      64    1024  1000    8   59.8    36.5   4 x 32
-//   fp8     128       8     0   20    6.4     4.9   a wave each
-//   fp8     128    1024  1000    8  140.7    56.9   a wave each
-//   fp8     128     512  1000    8   69.8    46.8   4 x 64
+//   fp8     128       8     0   20    6.4     5.1   a wave each
+//   fp8     128    1024  1000    8  140.7    56.5   a wave each
+//   fp8     128     512  1000    8   69.8    46.4   4 x 64
 //   fp8     128       8  4000  200  186.1   163.8   4 x 64
 //   fp8     128     256     0  200   68.7    51.3   4 x 64
 //   fp8     128     128  1000  200  127.0   (4 x 64: 136)  8 x 64

@@ -7,10 +7,12 @@
 //
 // A wave streams K/V for itself as the decode kernel does: K of the next
 // 32-token tile in registers, V through its own 8 KB of LDS, both as fp8, on
-// 16x16x32 MFMAs; two blocks of 16 columns use every tile.
+// 16x16x32 MFMAs; two blocks of 16 columns use every tile. Keys past the wave's
+// last token are not read; within the wave an infinite or NaN value row reaches
+// earlier tokens, as in prefill_attn.hip.
 //
 // Bound: the cache's bytes. 1024 pairs, 2 tokens after 2000, head_dim 128
-// (524 MB): 104 us; 8-wave workgroups sharing K/V 264 us (a round of 256
+// (524 MB): 105-108 us; 8-wave workgroups sharing K/V 264 us (a round of 256
 // pairs each), 2 waves on 32-key tiles 127 us.
 #include "attn_tiles.h"
 #include "tt_internal.h"
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(64, 2) void prefill_stream_kernel(PrefillArgs a) {
 
   // The decode kernel's pipeline: K(k + 1) | Q K^T, softmax | wait for V(k), read it | V(k + 1) | P V,
   // with explicit vmcnt counts (loads return in issue order). Every tile issues the next one's loads, the
-  // last of a span its own again: the counts, and no branch round the loads (with one, 143 us for 104 above).
+  // last of a span its own again: the counts, and no branch round the loads (with one, 143 us for 105 above).
   const int tiles = (L + kTileTokens - 1) / kTileTokens;
   for (int c0 = 0; c0 < tiles; c0 += kSpanTiles) {
     const int c1 = min(tiles, c0 + kSpanTiles);

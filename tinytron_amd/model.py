@@ -17,8 +17,7 @@ package's caches, a decode step (T = 1) is one split-K GQA attention launch
 pair that also applies RoPE to the step's token and appends it to the cache
 (fp32 caches: a RoPE + append kernel, then the attention kernels); prefill
 (T > 1) writes the cache with the RoPE + append kernel and attends with the
-prefill kernel (bf16 activations; SDPA per sequence for fp32). No CPU
-fallback.
+prefill kernels (bf16; fp32 over an fp32 cache). No CPU fallback.
 
 ``GPT.forward`` runs a bf16 decode step (T = 1) as a fused layer sequence
 when the shapes allow it (``GPT.fused_decode``): per layer, one skinny
@@ -189,8 +188,9 @@ class Attention(nn.Module):
     def _prefill(self, q, k, v, cache, table, lens_before):
         """T > 1: append all (ragged) prompt tokens with the fused kernel, then
         causal attention over each sequence's cached prefix (attn.py:321-341):
-        the prefill kernel for bf16 activations, row attention (one query row
-        per new token) for fp32 and the head dims that kernel does not take."""
+        the prefill kernels for bf16 activations and for fp32, row attention (one
+        query row per new token) for the head dims they do not take and, in
+        fp32, a few rows after a long prefix (PagedKVCache.prefill_attend)."""
         B, _, T, D = q.shape
         new = cache._pending_new_lens or [T] * B
         q_rot = cache.rope_append(q, k, v, table, new_lens=new)
